@@ -47,6 +47,35 @@ def test_fwht_scale_matches_oracle(cuda, d, block, batch):
     assert np.array_equal(got.view(np.uint16), ref16.view(np.uint16))
 
 
+@pytest.mark.parametrize("rows,d,block,ldz", [
+    (1, 4, 4, 8), (3, 4, 1, 4), (2, 1028, 4, 1280), (9, 1088, 64, 1280), (5, 6144, 2048, 6400), (7, 12288, 4096, 12288),
+    (4099, 2560, 512, 2560), (4097, 96, 2, 256), (1500, 3072, 1024, 3328), (520, 4096, 4096, 4096),
+    (2, 8192, 8192, 8448), (3, 1030, 2, 1280)])
+@pytest.mark.parametrize("post", [False, True])
+def test_rotated_rows_match_oracle(cuda, rows, d, block, ldz, post):
+    """tp_block_fwht_rows (with and without scales before and after) and
+    tp_fwht_scale_padded, one or several rows per wave, partial 1024- and
+    4096-column segments, one block per four columns up to 4096 and beyond,
+    rows of no multiple of 4: bit-exact with the oracle, zeros in the padding."""
+    from turbopress_amd import _lib
+    gen = torch.Generator().manual_seed(d + rows)
+    rs = ((torch.randn(d, generator=gen).sign()) * (torch.rand(d, generator=gen) + 0.5)).to(torch.float16)
+    x = (torch.randn(rows, d, generator=gen) * 3).to(torch.float16)
+    xd, rd = x.to(cuda), rs.to(cuda)
+    lib = _lib.lib()
+    if post:
+        out = torch.full((rows, d), float("nan"), dtype=torch.float16, device=cuda)
+        st = lib.tp_block_fwht_rows(xd.data_ptr(), 0, rd.data_ptr(), out.data_ptr(), rows, d, block, _stream())
+        ref = O.block_fwht(x.numpy().astype(np.float32), block) * rs.numpy().astype(np.float32)
+    else:
+        out = torch.full((rows, ldz), float("nan"), dtype=torch.float16, device=cuda)
+        st = lib.tp_fwht_scale_padded(xd.data_ptr(), rd.data_ptr(), out.data_ptr(), rows, d, block, ldz, _stream())
+        ref = np.zeros((rows, ldz), np.float32)
+        ref[:, :d] = O.block_fwht(x.numpy().astype(np.float32) * rs.numpy().astype(np.float32), block)
+    assert st == _lib.TP_OK
+    assert np.array_equal(out.cpu().numpy().view(np.uint16), ref.astype(np.float16).view(np.uint16))
+
+
 def test_fwht_scale_rejects_bad_block(cuda):
     from turbopress_amd.hip_kernel import fwht_scale
     x = torch.zeros(1, 96, dtype=torch.float16, device=cuda)
