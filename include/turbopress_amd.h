@@ -214,6 +214,23 @@ int tp_packed_linear_forward_noalloc(const uint16_t* x, int64_t ldx, int64_t bat
                                      const uint16_t* bias, int64_t n, int64_t d, int bits,
                                      int n_states, uint16_t* y, int64_t ldy, void* stream);
 
+/* Bytes of workspace tp_packed_linear_prefill needs (0 for sizes it does not
+ * take: batch outside [1, 65535], d above 2^20, n above 2^24).  Host only. */
+int64_t tp_prefill_workspace_bytes(int64_t n, int64_t d, int64_t batch, int bits);
+
+/* tp_packed_linear_forward for a whole prompt (meant for batch > 32): x
+ * (contiguous fp16 [batch, d]) is rotated once into the workspace (with
+ * rot_scale = NULL and block = 1: x is z already), then a GEMM decodes each
+ * weight tile once per 64..256 batch rows and feeds the matrix cores.  y: fp16
+ * [batch, ldy].  The workspace (16-byte aligned) may hold anything; the sums
+ * are added in a fixed order.
+ * Replaces turbopress/runtime.py:312-316 + 332-333 for prompt-sized inputs. */
+int tp_packed_linear_prefill(const uint16_t* x, int64_t batch, const uint16_t* rot_scale, int64_t block,
+                             const uint8_t* path_tiled, const uint8_t* member_tiled,
+                             const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias,
+                             int64_t n, int64_t d, int bits, int n_states, uint16_t* y, int64_t ldy,
+                             void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Host only: the cut the batch <= 8 one-pass kernel of
  * tp_packed_linear_forward / tp_packed_linear_forward_group takes for
  * n_linears linears of ns[i] rows sharing d columns (Hadamard block

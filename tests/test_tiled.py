@@ -189,6 +189,44 @@ def test_fused_forward_matches_oracle(cuda, n, d, bits, batch):
     assert O.max_rel(y, O.tiled_forward(payload_numpy(p), x.numpy())) <= GEMV_TOL
 
 
+# Prompt GEMM: one row tile and one column tile short of every tile the
+# planner takes (128 / 256 / 384 rows x 64 / 128 / 256 batch rows), one K part
+# and several (parts that start inside a row's path stream), a single segment
+# of K, rows of no multiple of 8 or 4, Hadamard blocks 2..8192.
+PREFILL_CASES = [  # n, d, bits, S, batch
+    (33, 64, 3, 64, 33), (17, 576, 2, 16, 40), (129, 320, 4, 4, 65), (1000, 1030, 3, 8, 67), (64, 8192, 3, 64, 40),
+    (306, 1280, 2, 64, 115), (1001, 2560, 3, 64, 130), (1536, 9728, 4, 64, 96), (2863, 5120, 3, 64, 193),
+    (3000, 1024, 3, 16, 1100), (4097, 768, 2, 4, 1000), (7000, 512, 4, 64, 1537), (9001, 64, 3, 64, 1500),
+]
+
+
+@pytest.mark.parametrize("n,d,bits,n_states,batch", PREFILL_CASES)
+def test_prompt_forward_matches_oracle_deterministically(cuda, n, d, bits, n_states, batch):
+    """forward and packed_gemv of more than 32 rows (tp_packed_linear_prefill)
+    against the fp64 product of the oracle's decoded weights and rotated
+    activations; a second call is bit-identical and writes nothing past y."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    p = make_payload(n, d, bits, n_states, seed=n + d, bias=bool(n % 2))
+    lin = PackedTCQLinear(p, mode="hip")
+    x = make_activation(batch, d, seed=batch)
+    pn = payload_numpy(p)
+    rs = O.rot_scale(pn["signs_packed"], pn["inv_equil"], d).astype(np.float32)
+    z = O.block_fwht(x.numpy().astype(np.float32) * rs, p["block"]).astype(np.float16)
+    w = torch.from_numpy(np.ascontiguousarray(O.decode_rows(pn, 0, n))).to(cuda).double()
+    ref = torch.from_numpy(z).to(cuda).double() @ w.T
+    yz = hk.packed_gemv(torch.from_numpy(z).to(cuda), lin)
+    assert O.max_rel(yz.float().cpu().numpy(), ref.cpu().numpy()) <= GEMV_TOL
+    if p["bias"] is not None:
+        ref = ref + p["bias"].to(cuda).double()
+    xd = x.to(cuda)
+    y = lin(xd)
+    assert O.max_rel(y.float().cpu().numpy(), ref.cpu().numpy()) <= GEMV_TOL
+    guard = torch.full((batch * n + 256,), 7.0, dtype=torch.float16, device=cuda)
+    out = guard[:batch * n].view(batch, n)
+    assert hk.forward_prefill(lin, xd, out, lin.bias)
+    assert torch.equal(out, y) and bool((guard[batch * n:] == 7.0).all())
+
+
 def test_fused_equals_two_launch_path(cuda):
     from turbopress_amd import hip_kernel as hk
     from turbopress_amd.runtime import PackedTCQLinear

@@ -54,6 +54,9 @@ SIGNATURES: dict[str, tuple] = {
                                          c_int, c_int, _P, _I64, _P, _I64, _P]),
     "tp_packed_linear_forward_noalloc": (c_int, [_P, _I64, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64,
                                                  c_int, c_int, _P, _I64, _P]),
+    "tp_prefill_workspace_bytes": (c_int64, [_I64, _I64, _I64, c_int]),
+    "tp_packed_linear_prefill": (c_int, [_P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64, c_int, c_int,
+                                         _P, _I64, _P, _I64, _P]),
     "tp_packed_linear_forward_group": (c_int, [c_int, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P,
                                                _I64, c_int, c_int, _P, _P, _P, _P, _P]),
 }

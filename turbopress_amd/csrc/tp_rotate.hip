@@ -22,6 +22,12 @@ namespace tp {
 
 constexpr int kRotMaxBlock = 16384;
 
+// Where the transformed rows go: row-major z [rows][ld], or the MFMA operand
+// order the prompt GEMM stages (tp_prefill.hip), `ld` columns per row.
+__device__ __forceinline__ size_t rot_out_index(bool packed, int64_t row, int64_t col, int64_t ld) {
+  return packed ? prefill_operand_index(row, col, ld >> 7) : (size_t)row * ld + col;
+}
+
 struct RotRows {
   const uint16_t* x;
   const uint16_t* pre;   // null: ones
@@ -30,6 +36,7 @@ struct RotRows {
   int64_t rows, groups;  // groups of `rpg` rows
   int32_t d, ld, rpg;
   float div, recip;
+  int32_t packed;
 };
 
 // One wave transforms 1024 columns of `rpg` consecutive rows, one after the
@@ -97,7 +104,7 @@ __global__ void __launch_bounds__(kRotThreads) rot_rows_kernel(const RotRows a) 
       } else {
         o = rot_z4<LOGH>(v + 4 * g, a.div, a.recip);
       }
-      gst(reinterpret_cast<u32x2_t*>(a.z + (r0 + r) * a.ld + col), o);
+      gst(reinterpret_cast<u32x2_t*>(a.z + rot_out_index(a.packed, r0 + r, col, a.ld)), o);
     }
   }
 }
@@ -114,7 +121,7 @@ template <int EPT>
 __global__ void __launch_bounds__(256)
 fwht_scale_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ rs,
                   const uint16_t* __restrict__ post, uint16_t* __restrict__ z, int64_t d,
-                  int64_t ldz, int block, float inv_norm_div) {
+                  int64_t ldz, int block, float inv_norm_div, bool packed) {
   extern __shared__ float buf[];
   const int64_t row = blockIdx.y;
   const int64_t base = (int64_t)blockIdx.x * block;
@@ -160,11 +167,11 @@ fwht_scale_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ r
   for (int i = t; i < block; i += blockDim.x) {
     float v = buf[i] / inv_norm_div;
     if (pr) v *= h2f(pr[i]);
-    z[row * ldz + base + i] = f2h(v);
+    z[rot_out_index(packed, row, base + i, ldz)] = f2h(v);
   }
   // The last block of a row also clears the padding columns [d, ldz).
   if (blockIdx.x == gridDim.x - 1) {
-    for (int64_t i = d + t; i < ldz; i += blockDim.x) z[row * ldz + i] = 0;
+    for (int64_t i = d + t; i < ldz; i += blockDim.x) z[rot_out_index(packed, row, i, ldz)] = 0;
   }
 }
 
@@ -173,7 +180,7 @@ fwht_scale_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ r
 namespace tp {
 
 int block_fwht(const uint16_t* x, const uint16_t* pre, const uint16_t* post, uint16_t* z,
-               int64_t rows, int64_t d, int64_t block, int64_t ldz, void* stream) {
+               int64_t rows, int64_t d, int64_t block, int64_t ldz, bool packed, void* stream) {
   if (!x || !z) return TP_ERR_NULL_POINTER;
   if (rows < 0 || d <= 0 || ldz < d) return TP_ERR_BAD_DIMS;
   if (block < 1 || (block & (block - 1)) || d % block || block > kRotMaxBlock) return TP_ERR_BAD_BLOCK;
@@ -197,6 +204,7 @@ int block_fwht(const uint16_t* x, const uint16_t* pre, const uint16_t* post, uin
     a.ld = (int32_t)ldz;
     a.div = div;
     a.recip = 1.f / div;
+    a.packed = packed;
     // rows per wave: one while the launch has fewer than 16 waves per CU
     const int64_t width = block > 1024 ? kRotTile : 1024, per = block > 1024 ? 4 : 1;
     const int64_t waves = (ldz + width - 1) / width * per * rows;
@@ -225,10 +233,10 @@ int block_fwht(const uint16_t* x, const uint16_t* pre, const uint16_t* post, uin
   dim3 grid((unsigned)(d / block), (unsigned)rows);
   const size_t lds = (size_t)block * sizeof(float);
   switch (ept) {
-    case 8: hipLaunchKernelGGL(fwht_scale_kernel<8>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div); break;
-    case 4: hipLaunchKernelGGL(fwht_scale_kernel<4>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div); break;
-    case 2: hipLaunchKernelGGL(fwht_scale_kernel<2>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div); break;
-    default: hipLaunchKernelGGL(fwht_scale_kernel<1>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div); break;
+    case 8: hipLaunchKernelGGL(fwht_scale_kernel<8>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div, packed); break;
+    case 4: hipLaunchKernelGGL(fwht_scale_kernel<4>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div, packed); break;
+    case 2: hipLaunchKernelGGL(fwht_scale_kernel<2>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div, packed); break;
+    default: hipLaunchKernelGGL(fwht_scale_kernel<1>, grid, dim3(threads), lds, s, x, pre, post, z, d, ldz, (int)block, div, packed); break;
   }
   return launch_status();
 }
@@ -238,18 +246,18 @@ int block_fwht(const uint16_t* x, const uint16_t* pre, const uint16_t* post, uin
 extern "C" int tp_fwht_scale(const uint16_t* x, const uint16_t* rot_scale, uint16_t* z,
                              int64_t batch, int64_t d, int64_t block, void* stream) {
   if (!rot_scale) return TP_ERR_NULL_POINTER;
-  return tp::block_fwht(x, rot_scale, nullptr, z, batch, d, block, d, stream);
+  return tp::block_fwht(x, rot_scale, nullptr, z, batch, d, block, d, false, stream);
 }
 
 extern "C" int tp_fwht_scale_padded(const uint16_t* x, const uint16_t* rot_scale, uint16_t* z,
                                     int64_t batch, int64_t d, int64_t block, int64_t ldz,
                                     void* stream) {
   if (!rot_scale) return TP_ERR_NULL_POINTER;
-  return tp::block_fwht(x, rot_scale, nullptr, z, batch, d, block, ldz, stream);
+  return tp::block_fwht(x, rot_scale, nullptr, z, batch, d, block, ldz, false, stream);
 }
 
 extern "C" int tp_block_fwht_rows(const uint16_t* x, const uint16_t* pre_scale,
                                   const uint16_t* post_scale, uint16_t* out,
                                   int64_t rows, int64_t d, int64_t block, void* stream) {
-  return tp::block_fwht(x, pre_scale, post_scale, out, rows, d, block, d, stream);
+  return tp::block_fwht(x, pre_scale, post_scale, out, rows, d, block, d, false, stream);
 }

@@ -190,37 +190,49 @@ template <> struct TrellisOf<8> { static constexpr int m = 3; static constexpr u
 template <> struct TrellisOf<16> { static constexpr int m = 4; static constexpr uint32_t g0 = 023, g1 = 035; };
 template <> struct TrellisOf<64> { static constexpr int m = 6; static constexpr uint32_t g0 = 0133, g1 = 0171; };
 
-// Subset words of the two 16-weight groups carried by one interleaved path word.
+// Subset words of the two 16-weight groups carried by one interleaved path
+// word, in two steps: the delayed path words, then
 // SA bit 2j / 2j+1 = subset bit 0 / 1 of first-half weight j; SB likewise for
 // the second half.  `prev` is the interleaved word of the 16 preceding columns
 // of each half.
 template <int NS>
-__device__ __forceinline__ void subset_words(uint32_t cur, uint32_t prev, uint32_t& SA, uint32_t& SB) {
-  constexpr int m = TrellisOf<NS>::m;
-  constexpr uint32_t D0 = delay_mask(TrellisOf<NS>::g0, m);
-  constexpr uint32_t D1 = delay_mask(TrellisOf<NS>::g1, m);
+struct SubsetTaps {
+  static constexpr int m = TrellisOf<NS>::m;
   uint32_t sh[m + 1];
-  sh[0] = cur;
+  __device__ __forceinline__ void shift(uint32_t cur, uint32_t prev) {
+    sh[0] = cur;
 #pragma unroll
-  for (int t = 1; t <= m; ++t) sh[t] = __builtin_amdgcn_alignbit(cur, prev, 32 - 2 * t);
-  uint32_t e0, e1;
-  if constexpr (NS == 64) {
-    // taps {0,1,2,4,5} and {0,1,4,5,6}: shared part first, three-input XORs
-    static_assert(D0 == 0x37u && D1 == 0x73u, "S=64 generator taps");
-    const uint32_t c = __builtin_amdgcn_bitop3_b32(sh[0], sh[1], sh[4], 0x96);
-    e0 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[2], 0x96);
-    e1 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[6], 0x96);
-  } else {
-    e0 = 0u;
-    e1 = 0u;
-#pragma unroll
-    for (int t = 0; t <= m; ++t) {
-      if ((D0 >> t) & 1u) e0 ^= sh[t];
-      if ((D1 >> t) & 1u) e1 ^= sh[t];
-    }
+    for (int t = 1; t <= m; ++t) sh[t] = __builtin_amdgcn_alignbit(cur, prev, 32 - 2 * t);
   }
-  SA = (e0 & 0x55555555u) | ((e1 << 1) & 0xAAAAAAAAu);
-  SB = ((e0 >> 1) & 0x55555555u) | (e1 & 0xAAAAAAAAu);
+  __device__ __forceinline__ void words(uint32_t& SA, uint32_t& SB) const {
+    constexpr uint32_t D0 = delay_mask(TrellisOf<NS>::g0, m);
+    constexpr uint32_t D1 = delay_mask(TrellisOf<NS>::g1, m);
+    uint32_t e0, e1;
+    if constexpr (NS == 64) {
+      // taps {0,1,2,4,5} and {0,1,4,5,6}: shared part first, three-input XORs
+      static_assert(D0 == 0x37u && D1 == 0x73u, "S=64 generator taps");
+      const uint32_t c = __builtin_amdgcn_bitop3_b32(sh[0], sh[1], sh[4], 0x96);
+      e0 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[2], 0x96);
+      e1 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[6], 0x96);
+    } else {
+      e0 = 0u;
+      e1 = 0u;
+#pragma unroll
+      for (int t = 0; t <= m; ++t) {
+        if ((D0 >> t) & 1u) e0 ^= sh[t];
+        if ((D1 >> t) & 1u) e1 ^= sh[t];
+      }
+    }
+    SA = (e0 & 0x55555555u) | ((e1 << 1) & 0xAAAAAAAAu);
+    SB = ((e0 >> 1) & 0x55555555u) | (e1 & 0xAAAAAAAAu);
+  }
+};
+
+template <int NS>
+__device__ __forceinline__ void subset_words(uint32_t cur, uint32_t prev, uint32_t& SA, uint32_t& SB) {
+  SubsetTaps<NS> taps;
+  taps.shift(cur, prev);
+  taps.words(SA, SB);
 }
 
 // LDS byte address of the lane's copy of table entry `byte b of idx` in
@@ -277,6 +289,71 @@ __device__ __forceinline__ void split_members(const W& w, MemberWords<KB> m[2]) 
   }
 }
 
+// Table index words of 32 weights (16 of each half) of one lane: w[0..1] the
+// even / odd pairs of the first half, w[2..3] of the second; k=4 also the
+// lane-offset words with the pairs' high member bits, l[i] for w[i].
+template <int KB>
+struct DecodeIndex {
+  uint32_t w[4];
+  uint32_t l[KB == 4 ? 4 : 1];
+};
+
+template <int KB>
+__device__ __forceinline__ DecodeIndex<KB> pair_index(uint32_t SA, uint32_t SB, const MemberWords<KB>& M,
+                                                      uint32_t laneoff) {
+  DecodeIndex<KB> d;
+  if constexpr (KB == 4) {
+    // One table format: index byte [S0a S1a S0b S1b | M0a M1a M0b M1b] of the
+    // low member bits (odd pairs shifted into place), the pair's two high
+    // member bits into bits 6..7 of the lane-offset byte (row within the
+    // index byte's 256-byte group).
+    d.w[0] = (SA & 0x0F0F0F0Fu) | (M.a & 0xF0F0F0F0u);
+    d.w[1] = ((SA >> 4) & 0x0F0F0F0Fu) | ((M.a << 4) & 0xF0F0F0F0u);
+    d.w[2] = (SB & 0x0F0F0F0Fu) | (M.b & 0xF0F0F0F0u);
+    d.w[3] = ((SB >> 4) & 0x0F0F0F0Fu) | ((M.b << 4) & 0xF0F0F0F0u);
+    d.l[0] = (M.q & 0xC0C0C0C0u) | laneoff;
+    d.l[1] = ((M.q << 2) & 0xC0C0C0C0u) | laneoff;
+    d.l[2] = ((M.q << 4) & 0xC0C0C0C0u) | laneoff;
+    d.l[3] = ((M.q << 6) & 0xC0C0C0C0u) | laneoff;
+  } else if constexpr (KB == 3) {
+    // Member words are stored nibble-swapped within each byte, so one bit
+    // select pairs every subset nibble with its member nibble: even pairs as
+    // [subset | member << 4] (format 0), odd pairs as [member | subset << 4]
+    // (format 1).
+    d.w[0] = (SA & 0x0F0F0F0Fu) | (M.a & 0xF0F0F0F0u);
+    d.w[1] = (SA & 0xF0F0F0F0u) | (M.a & 0x0F0F0F0Fu);
+    d.w[2] = (SB & 0x0F0F0F0Fu) | (M.b & 0xF0F0F0F0u);
+    d.w[3] = (SB & 0xF0F0F0F0u) | (M.b & 0x0F0F0F0Fu);
+    d.l[0] = laneoff;
+  } else {
+    d.w[0] = (SA & 0x0F0F0F0Fu) | ((M.w << 4) & 0xF0F0F0F0u);
+    d.w[1] = ((SA >> 4) & 0x0F0F0F0Fu) | (M.w & 0xF0F0F0F0u);
+    d.w[2] = (SB & 0x0F0F0F0Fu) | ((M.w << 2) & 0xF0F0F0F0u);
+    d.w[3] = ((SB >> 4) & 0x0F0F0F0Fu) | ((M.w >> 2) & 0xF0F0F0F0u);
+    d.l[0] = laneoff;
+  }
+  return d;
+}
+
+// Word v (0..3) of MFMA A operand j (0..3) of an indexed word: operands j =
+// 0 / 1 are first-half columns 0-7 / 8-15, j = 2 / 3 the second half's.
+template <int KB>
+__device__ __forceinline__ uint32_t decode_lookup_word(const DecodeIndex<KB>& d, const uint32_t* table, int j, int v) {
+  constexpr int FO = KB == 3 ? 1 : 0;  // table format of the odd-pair index words
+  const int e = (j & 2) + (v & 1);     // index word: this half's even or odd pairs
+  const int b = 2 * (j & 1) + (v >> 1);
+  if constexpr (KB == 4) return lds_word(table, table_addr4(d.w[e], d.l[e], b));
+  else return (v & 1) ? lds_word(table, table_addr<FO>(d.w[e], d.l[0], b)) : lds_word(table, table_addr<0>(d.w[e], d.l[0], b));
+}
+
+template <int KB>
+__device__ __forceinline__ u32x4_t decode_lookup(const DecodeIndex<KB>& d, const uint32_t* table, int j) {
+  u32x4_t A;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) A[v] = decode_lookup_word<KB>(d, table, j, v);
+  return A;
+}
+
 // Decode 32 weights (16 of each half) of one lane into four MFMA A operands:
 // A[0]/A[1] = first-half columns 0-7 / 8-15, A[2]/A[3] = second half.
 template <int KB, int NS>
@@ -284,58 +361,13 @@ __device__ __forceinline__ void decode_word(uint32_t cur, uint32_t prev, const M
                                             const uint32_t* table, uint32_t laneoff, u32x4_t A[4]) {
   uint32_t SA, SB;
   subset_words<NS>(cur, prev, SA, SB);
-  if constexpr (KB == 4) {
-    // One table format: index byte [S0a S1a S0b S1b | M0a M1a M0b M1b] of the
-    // low member bits (odd pairs shifted into place), the pair's two high
-    // member bits into bits 6..7 of the lane-offset byte (row within the
-    // index byte's 256-byte group).
-    const uint32_t iae = (SA & 0x0F0F0F0Fu) | (M.a & 0xF0F0F0F0u);
-    const uint32_t iao = ((SA >> 4) & 0x0F0F0F0Fu) | ((M.a << 4) & 0xF0F0F0F0u);
-    const uint32_t ibe = (SB & 0x0F0F0F0Fu) | (M.b & 0xF0F0F0F0u);
-    const uint32_t ibo = ((SB >> 4) & 0x0F0F0F0Fu) | ((M.b << 4) & 0xF0F0F0F0u);
-    const uint32_t lae = (M.q & 0xC0C0C0C0u) | laneoff;
-    const uint32_t lao = ((M.q << 2) & 0xC0C0C0C0u) | laneoff;
-    const uint32_t lbe = ((M.q << 4) & 0xC0C0C0C0u) | laneoff;
-    const uint32_t lbo = ((M.q << 6) & 0xC0C0C0C0u) | laneoff;
+  const DecodeIndex<KB> d = pair_index<KB>(SA, SB, M, laneoff);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      A[0][2 * h] = lds_word(table, table_addr4(iae, lae, h));
-      A[0][2 * h + 1] = lds_word(table, table_addr4(iao, lao, h));
-      A[1][2 * h] = lds_word(table, table_addr4(iae, lae, 2 + h));
-      A[1][2 * h + 1] = lds_word(table, table_addr4(iao, lao, 2 + h));
-      A[2][2 * h] = lds_word(table, table_addr4(ibe, lbe, h));
-      A[2][2 * h + 1] = lds_word(table, table_addr4(ibo, lbo, h));
-      A[3][2 * h] = lds_word(table, table_addr4(ibe, lbe, 2 + h));
-      A[3][2 * h + 1] = lds_word(table, table_addr4(ibo, lbo, 2 + h));
-    }
-  } else {
-    uint32_t iae, iao, ibe, ibo;
-    constexpr int FO = KB == 3 ? 1 : 0;  // table format of the odd-pair index words
-    if constexpr (KB == 3) {
-      // Member words are stored nibble-swapped within each byte, so one bit
-      // select pairs every subset nibble with its member nibble: even pairs as
-      // [subset | member << 4] (format 0), odd pairs as [member | subset << 4]
-      // (format 1).
-      iae = (SA & 0x0F0F0F0Fu) | (M.a & 0xF0F0F0F0u);
-      iao = (SA & 0xF0F0F0F0u) | (M.a & 0x0F0F0F0Fu);
-      ibe = (SB & 0x0F0F0F0Fu) | (M.b & 0xF0F0F0F0u);
-      ibo = (SB & 0xF0F0F0F0u) | (M.b & 0x0F0F0F0Fu);
-    } else {
-      iae = (SA & 0x0F0F0F0Fu) | ((M.w << 4) & 0xF0F0F0F0u);
-      iao = ((SA >> 4) & 0x0F0F0F0Fu) | (M.w & 0xF0F0F0F0u);
-      ibe = (SB & 0x0F0F0F0Fu) | ((M.w << 2) & 0xF0F0F0F0u);
-      ibo = ((SB >> 4) & 0x0F0F0F0Fu) | ((M.w >> 2) & 0xF0F0F0F0u);
-    }
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      A[0][2 * h] = lds_word(table, table_addr<0>(iae, laneoff, h));
-      A[0][2 * h + 1] = lds_word(table, table_addr<FO>(iao, laneoff, h));
-      A[1][2 * h] = lds_word(table, table_addr<0>(iae, laneoff, 2 + h));
-      A[1][2 * h + 1] = lds_word(table, table_addr<FO>(iao, laneoff, 2 + h));
-      A[2][2 * h] = lds_word(table, table_addr<0>(ibe, laneoff, h));
-      A[2][2 * h + 1] = lds_word(table, table_addr<FO>(ibo, laneoff, h));
-      A[3][2 * h] = lds_word(table, table_addr<0>(ibe, laneoff, 2 + h));
-      A[3][2 * h + 1] = lds_word(table, table_addr<FO>(ibo, laneoff, 2 + h));
+    for (int j = 0; j < 4; ++j) {
+      A[j][2 * h] = decode_lookup_word<KB>(d, table, j, 2 * h);
+      A[j][2 * h + 1] = decode_lookup_word<KB>(d, table, j, 2 * h + 1);
     }
   }
 }
@@ -714,6 +746,23 @@ constexpr int kLinearNotHandled = 1 << 20;
 int linear_forward_fast(const TiledLinearArgs* ls, int n_lin, int64_t batch, const uint16_t* codebook,
                         int bits, int n_states, hipStream_t s, bool clear_ws);
 int64_t linear_ksplit_bytes(int64_t T);
+
+// z = blockFWHT(x * pre) * post of `rows` rows (tp_rotate.hip; null scales:
+// ones), row-major with row stride ldz and zeros in [d, ldz), or with
+// `packed` in the operand order below, ldz = 128 U columns per row.
+int block_fwht(const uint16_t* x, const uint16_t* pre, const uint16_t* post, uint16_t* z, int64_t rows, int64_t d,
+               int64_t block, int64_t ldz, bool packed, void* stream);
+
+// Operand order of the prompt GEMM's activations: element (b, c) of a z of
+// 128 U columns.  A block of 1024 bytes is one v_mfma_f32_32x32x16_f16
+// operand as its 64 lanes read it: lane l holds 8 columns of batch row
+// 32 (b / 32) + l % 32 in segment 2 u + l / 32, from mfma_col(4 x + j) on.
+// Blocks are ordered [b / 32][u][x][j].
+__host__ __device__ inline size_t prefill_operand_index(int64_t b, int64_t c, int64_t U) {
+  const int cc = (int)(c & 63), x = (cc >> 4) & 1, j = ((cc >> 5) & 1) * 2 + ((cc >> 3) & 1);
+  const int lane = (int)(b & 31) + 32 * (int)((c >> 6) & 1);
+  return (size_t)(((((b >> 5) * U + (c >> 7)) * 2 + x) * 4 + j) * 64 + lane) * 8 + (cc & 7);
+}
 
 // Zero `bytes` (a multiple of 4) of device memory with a fill kernel on
 // stream s (a kernel node rather than a memset node under graph capture).

@@ -120,6 +120,9 @@ def packed_gemv(z: Tensor, layer, bias: Tensor | None = None) -> Tensor:
     flat = z.reshape(-1, d).to(torch.float16).contiguous()
     out = torch.empty(flat.shape[0], n, dtype=torch.float16, device=z.device)
     if getattr(layer, "tiled_packed", None) is not None:
+        # (rows of no multiple of 4 columns would be laid out column by column)
+        if flat.shape[0] > 32 and d % 4 == 0 and forward_prefill(layer, flat, out, bias, rotated=True):
+            return out.reshape(*z.shape[:-1], n)
         ldz = layer._tiled_geo["z_cols"]
         zpad = flat if ldz == d else torch.nn.functional.pad(flat, (0, ldz - d))
         gemv_tiled(zpad, layer, bias, out)
@@ -275,16 +278,49 @@ def gemv_tiled(zpad: Tensor, layer, bias: Tensor | None, out: Tensor) -> Tensor:
     return out
 
 
+_PREFILL_ROWS = 32768  # rows per prompt GEMM (bounds its workspace)
+
+
+def forward_prefill(layer, flat: Tensor, y: Tensor, bias: Tensor | None, rotated: bool = False) -> bool:
+    """y = forward of more than 32 rows `flat` (contiguous fp16 [B, d]; with
+    `rotated` they are z already) by the prompt GEMM (tp_packed_linear_prefill);
+    False for sizes it does not take."""
+    n, d = layer.out_features, layer.in_features
+    rot, block = (0, 1) if rotated else (layer.rot_scale.data_ptr(), layer.block)
+    lib = _lib.lib()
+    rows = flat.shape[0]
+    need = int(lib.tp_prefill_workspace_bytes(n, d, min(rows, _PREFILL_ROWS), layer.bits))
+    if need <= 0:
+        return False
+    ws = None
+    buf = layer.tiled_packed
+    stream = current_stream_ptr(flat.device)
+    for b0 in range(0, rows, _PREFILL_ROWS):
+        nb = min(_PREFILL_ROWS, rows - b0)
+        need = int(lib.tp_prefill_workspace_bytes(n, d, nb, layer.bits))
+        if ws is None or ws.numel() < need:
+            ws = torch.empty(need, dtype=torch.uint8, device=flat.device)
+        st = lib.tp_packed_linear_prefill(
+            flat.data_ptr() + 2 * b0 * d, nb, rot, block, buf.data_ptr(),
+            buf.data_ptr() + layer._tiled_geo["path_bytes"], layer.scales.data_ptr(),
+            layer.codebook.data_ptr(), 0 if bias is None else bias.data_ptr(), n, d, layer.bits,
+            layer.n_states, y.data_ptr() + 2 * b0 * n, n, ws.data_ptr(), ws.numel(), stream)
+        _lib.check(st, "packed_linear_prefill")
+    return True
+
+
 def forward_tiled(layer, x: Tensor) -> Tensor:
-    """Rotation + decode-GEMV + bias: one fused launch per 32 rows
-    (tp_packed_linear_forward) when the rotation fits the launch (up to 8
-    rows, or Hadamard blocks <= 512); otherwise the rows rotate once into the
-    padded layout and run the batched decode-GEMV (tp_tcq_gemv_tiled) per 32
-    rows.  fp16 [..., n]."""
+    """Rotation + decode-GEMV + bias: more than 32 rows run the prompt GEMM
+    (forward_prefill); up to 32 one fused launch (tp_packed_linear_forward)
+    when the rotation fits the launch (up to 8 rows, or Hadamard blocks <=
+    512), otherwise the rows rotate once into the padded layout and run the
+    batched decode-GEMV (tp_tcq_gemv_tiled).  fp16 [..., n]."""
     _require_cuda(x, "x")
     n, d = layer.out_features, layer.in_features
     flat = x.reshape(-1, d).to(torch.float16).contiguous()
     y = torch.empty(flat.shape[0], n, dtype=torch.float16, device=x.device)
+    if flat.shape[0] > 32 and forward_prefill(layer, flat, y, layer.bias):
+        return y.reshape(*x.shape[:-1], n)
     if d % 4 or (flat.shape[0] > 8 and (layer.block > 512 or d % 8)):
         # Rows not 8-byte aligned, or a batch whose Hadamard blocks span more
         # than one 512-column chunk: rotate into the padded layout, then GEMV.
