@@ -251,12 +251,10 @@ tcq_prefill_kernel(const PrefillArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[g][c][i] = 0.f;
 
-  // Index words of half step x of group g from its loaded words, in four
-  // chunks of a few instructions (run between MFMAs).
+  // Index words of half step x of group g from its loaded words, in three
+  // chunks of a few instructions (run between MFMAs; q = 2 is left empty).
   DecodeIndex<KB> idx[2][MG];
-  uint32_t prevw = 0;
-  SubsetTaps<NS> taps;
-  uint32_t SA = 0, SB = 0;
+  uint32_t prevw = 0, SA = 0, SB = 0;
   auto chunk = [&](auto xc, int g, int q) __attribute__((always_inline)) {
     constexpr int x = decltype(xc)::value;
     if (q == 0) {
@@ -269,10 +267,8 @@ tcq_prefill_kernel(const PrefillArgs a) {
         prevw = X[g][0];
       }
     } else if (q == 1) {
-      taps.shift(X[g][x], prevw);
-    } else if (q == 2) {
-      taps.words(SA, SB);
-    } else {
+      subset_words<NS>(X[g][x], prevw, SA, SB);
+    } else if (q == 3) {
       MemberWords<KB> m[2];
       split_members<KB>(M[g], m);
       idx[x][g] = pair_index<KB>(SA, SB, m[x], laneoff);

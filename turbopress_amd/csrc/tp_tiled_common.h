@@ -190,49 +190,37 @@ template <> struct TrellisOf<8> { static constexpr int m = 3; static constexpr u
 template <> struct TrellisOf<16> { static constexpr int m = 4; static constexpr uint32_t g0 = 023, g1 = 035; };
 template <> struct TrellisOf<64> { static constexpr int m = 6; static constexpr uint32_t g0 = 0133, g1 = 0171; };
 
-// Subset words of the two 16-weight groups carried by one interleaved path
-// word, in two steps: the delayed path words, then
+// Subset words of the two 16-weight groups carried by one interleaved path word.
 // SA bit 2j / 2j+1 = subset bit 0 / 1 of first-half weight j; SB likewise for
 // the second half.  `prev` is the interleaved word of the 16 preceding columns
 // of each half.
 template <int NS>
-struct SubsetTaps {
-  static constexpr int m = TrellisOf<NS>::m;
-  uint32_t sh[m + 1];
-  __device__ __forceinline__ void shift(uint32_t cur, uint32_t prev) {
-    sh[0] = cur;
-#pragma unroll
-    for (int t = 1; t <= m; ++t) sh[t] = __builtin_amdgcn_alignbit(cur, prev, 32 - 2 * t);
-  }
-  __device__ __forceinline__ void words(uint32_t& SA, uint32_t& SB) const {
-    constexpr uint32_t D0 = delay_mask(TrellisOf<NS>::g0, m);
-    constexpr uint32_t D1 = delay_mask(TrellisOf<NS>::g1, m);
-    uint32_t e0, e1;
-    if constexpr (NS == 64) {
-      // taps {0,1,2,4,5} and {0,1,4,5,6}: shared part first, three-input XORs
-      static_assert(D0 == 0x37u && D1 == 0x73u, "S=64 generator taps");
-      const uint32_t c = __builtin_amdgcn_bitop3_b32(sh[0], sh[1], sh[4], 0x96);
-      e0 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[2], 0x96);
-      e1 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[6], 0x96);
-    } else {
-      e0 = 0u;
-      e1 = 0u;
-#pragma unroll
-      for (int t = 0; t <= m; ++t) {
-        if ((D0 >> t) & 1u) e0 ^= sh[t];
-        if ((D1 >> t) & 1u) e1 ^= sh[t];
-      }
-    }
-    SA = (e0 & 0x55555555u) | ((e1 << 1) & 0xAAAAAAAAu);
-    SB = ((e0 >> 1) & 0x55555555u) | (e1 & 0xAAAAAAAAu);
-  }
-};
-
-template <int NS>
 __device__ __forceinline__ void subset_words(uint32_t cur, uint32_t prev, uint32_t& SA, uint32_t& SB) {
-  SubsetTaps<NS> taps;
-  taps.shift(cur, prev);
-  taps.words(SA, SB);
+  constexpr int m = TrellisOf<NS>::m;
+  constexpr uint32_t D0 = delay_mask(TrellisOf<NS>::g0, m);
+  constexpr uint32_t D1 = delay_mask(TrellisOf<NS>::g1, m);
+  uint32_t sh[m + 1];
+  sh[0] = cur;
+#pragma unroll
+  for (int t = 1; t <= m; ++t) sh[t] = __builtin_amdgcn_alignbit(cur, prev, 32 - 2 * t);
+  uint32_t e0, e1;
+  if constexpr (NS == 64) {
+    // taps {0,1,2,4,5} and {0,1,4,5,6}: shared part first, three-input XORs
+    static_assert(D0 == 0x37u && D1 == 0x73u, "S=64 generator taps");
+    const uint32_t c = __builtin_amdgcn_bitop3_b32(sh[0], sh[1], sh[4], 0x96);
+    e0 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[2], 0x96);
+    e1 = __builtin_amdgcn_bitop3_b32(c, sh[5], sh[6], 0x96);
+  } else {
+    e0 = 0u;
+    e1 = 0u;
+#pragma unroll
+    for (int t = 0; t <= m; ++t) {
+      if ((D0 >> t) & 1u) e0 ^= sh[t];
+      if ((D1 >> t) & 1u) e1 ^= sh[t];
+    }
+  }
+  SA = (e0 & 0x55555555u) | ((e1 << 1) & 0xAAAAAAAAu);
+  SB = ((e0 >> 1) & 0x55555555u) | (e1 & 0xAAAAAAAAu);
 }
 
 // LDS byte address of the lane's copy of table entry `byte b of idx` in
