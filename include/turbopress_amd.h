@@ -346,7 +346,7 @@ int tp_decode_tiled(const uint8_t* path_tiled, const uint8_t* member_tiled,
  * TCQ encoder (compress time)
  * ------------------------------------------------------------------------- */
 
-/* Workspace of tp_tcq_viterbi: one 64-bit branch-decision word per column
+/* Workspace of tp_tcq_viterbi: at most 64 branch-decision bits per column
  * and row (n * d * 8 bytes).  Host only. */
 int64_t tp_viterbi_workspace_bytes(int64_t n, int64_t d);
 

@@ -93,6 +93,27 @@ def test_viterbi_long_rows_and_odd_sizes(cuda):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_states", [4, 8, 16, 64])
+@pytest.mark.parametrize("d", [2, 31, 32, 33, 64, 95, 96, 97, 128, 191, 192, 193, 224, 320])
+def test_viterbi_block_edges(cuda, n_states, d):
+    """Row lengths around the 32-column history words and the 96-column blocks
+    (every column phase at the end of a row), values that overflow to infinite
+    metrics among them: bit-exact with the oracle's search."""
+    from turbopress_amd.encoder import viterbi
+    gen = torch.Generator().manual_seed(d)
+    cb = lloyd_max_gaussian(4)[0].to(torch.float32)
+    z = torch.randn(6, d, generator=gen)
+    z[1, d // 2] = 1e30
+    z[2, d - 1] = -1e30
+    z[3, d // 3] = float("inf")
+    start = torch.randint(0, n_states, (6,), generator=gen)
+    want = viterbi_full(z, cb, n_states, start)
+    got = viterbi(z.to(cuda), cb, n_states, start)
+    for w, g, name in zip(want, got, ("level", "path", "member", "end")):
+        assert torch.equal(g.cpu().to(w.dtype), w), name
+
+
+@pytest.mark.gpu
 def test_gpu_quantizer_round_trip_and_distortion(cuda):
     """tests/test_trellis.py:29-61: the stored bits rebuild the level codes,
     and 8-state TCQ at 2 bits beats the scalar Lloyd-Max optimum on N(0,1)
