@@ -111,6 +111,35 @@ def test_decode_rows_bit_exact(cuda, n, d, bits, n_states):
         assert np.array_equal(got.view(np.uint16), ref.view(np.uint16)), (r0, r1)
 
 
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("n,d,n_states", [(1, 1, 64), (3, 7, 4), (2, 9, 64), (37, 63, 16), (5, 512, 64), (6, 520, 8),
+                                          (4, 1031, 64), (70, 64, 64)])
+def test_decode_natural_streams_at_every_rate(cuda, n, d, bits, n_states):
+    """tp_decode_rows and tp_window_decode_levels, 8 columns per thread: rows
+    ending inside a byte of either stream, one to several 512-column spans,
+    wide and element stores (out strides of no multiple of 8), a row slice."""
+    from turbopress_amd import _lib
+    p = make_payload(n, d, bits, n_states, seed=n + d + bits)
+    pn = payload_numpy(p)
+    path = p["path_packed"].to(cuda)
+    mem = None if p["member_packed"] is None else p["member_packed"].to(cuda)
+    scales, cb = p["scales"].to(cuda), p["codebook"].to(cuda)
+    mp, ms = (0, 0) if mem is None else (mem.data_ptr(), mem.stride(0))
+    lib = _lib.lib()
+    for stride in (d, (d + 7) // 8 * 8 + 8, d + 3):
+        w = torch.full((n, stride), 7.0, dtype=torch.float16, device=cuda)
+        lev = torch.full((n, stride), 255, dtype=torch.uint8, device=cuda)
+        r0 = n // 2
+        assert lib.tp_decode_rows(path[r0:].data_ptr(), path.stride(0), mp + r0 * ms, ms, scales[r0:].data_ptr(),
+                                  cb.data_ptr(), n - r0, d, bits, n_states, w[r0:].data_ptr(), stride,
+                                  _stream()) == _lib.TP_OK
+        assert lib.tp_window_decode_levels(path.data_ptr(), path.stride(0), mp, ms, n, d, bits, n_states,
+                                           lev.data_ptr(), stride, _stream()) == _lib.TP_OK
+        assert np.array_equal(lev[:, :d].cpu().numpy(), O.levels_of(pn)) and bool((lev[:, d:] == 255).all())
+        assert np.array_equal(w[r0:, :d].cpu().numpy().view(np.uint16), O.decode_rows(pn, r0, n).view(np.uint16))
+        assert bool((w[:r0] == 7.0).all()) and bool((w[:, d:] == 7.0).all())
+
+
 # ---------------------------------------------------------------------- GEMV
 GEMV_CASES = [
     # (n, d, bits, n_states, batch)

@@ -29,6 +29,9 @@ DECODE_CASES = [
 ]
 
 
+DECODE_CASES += [(n, d, k, 64) for k in (2, 3, 4) for n, d in ((1, 1), (3, 63), (18, 65), (2, 71), (4, 255), (5, 257))]
+
+
 @pytest.mark.parametrize("n,d,bits,n_states", DECODE_CASES)
 def test_tiled_decode_bit_exact(cuda, n, d, bits, n_states):
     from turbopress_amd.runtime import PackedTCQLinear

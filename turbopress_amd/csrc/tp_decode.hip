@@ -7,11 +7,11 @@
 //                           factored out of an fp32 reduction, fp16 output)
 //                           then the fp16 bias add of runtime.py:332-333.
 //
-// These kernels read the streams exactly as the reference stores them (one
-// weight per thread, byte-granular little-endian field reads), support every
-// bits in [1, 7] and every S in {4, 8, 16, 64}, and serve as the bit-exact
-// decode entry points and the general fallback GEMV.  The bandwidth-tuned
-// path for k in {2, 3, 4} lives in tp_gemv_tiled.hip.
+// These kernels read the streams exactly as the reference stores them (byte-
+// granular little-endian field reads), support every bits in [1, 7] and every
+// S in {4, 8, 16, 64}, and serve as the bit-exact decode entry points and the
+// general fallback GEMV.  The bandwidth-tuned path for k in {2, 3, 4} lives in
+// tp_tiled.hip, tp_linear.hip, tp_stack.hip and tp_prefill.hip.
 #include "tp_common.h"
 
 namespace tp {
@@ -40,23 +40,101 @@ __device__ __forceinline__ uint32_t level_at(const DecodeArgs& a, int64_t r, int
   return mem * 4u + sub;
 }
 
-__global__ void window_decode_kernel(DecodeArgs a, uint8_t* __restrict__ out, int64_t out_stride) {
-  const int64_t r = blockIdx.y;
-  for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.d;
-       c += (int64_t)gridDim.x * blockDim.x) {
-    out[r * out_stride + c] = (uint8_t)level_at(a, r, c);
+// The 8 columns from c (a multiple of 8) of row r: their path bits are byte
+// c / 8 of the row, the up to 6 bits before them the byte before it (zero at
+// the row's start), their members the bits - 1 bytes from c / 8 * (bits - 1)
+// on.  Both subset bits of all 8 are XORs of the two path bytes shifted by the
+// generators' taps (dm0, dm1: bit t set where the subset bit takes the path
+// bit t columns back).  level[j] past the row's end is whatever zero stream
+// bits decode to.
+template <int BITS>
+__device__ __forceinline__ void levels_of_8(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, int64_t r, int64_t c,
+                                            uint32_t level[8]) {
+  const int64_t byte = c >> 3;
+  const uint8_t* prow = a.path + r * a.path_stride + byte;
+  const uint32_t p = ((uint32_t)prow[0] << 8) | (byte > 0 ? (uint32_t)prow[-1] : 0u);
+  uint32_t e0 = 0, e1 = 0;
+#pragma unroll
+  for (int t = 0; t <= 6; ++t) {
+    e0 ^= (p << t) & (0u - ((dm0 >> t) & 1u));
+    e1 ^= (p << t) & (0u - ((dm1 >> t) & 1u));
+  }
+  constexpr int mb = BITS - 1;
+  uint64_t mem = 0;  // 8 * mb bits
+  if constexpr (mb > 0) {
+    const uint8_t* mrow = a.member + r * a.member_stride;
+    const int64_t m0 = byte * mb, mend = (a.d * mb + 7) >> 3;
+    if (c + 8 <= a.d) {
+#pragma unroll
+      for (int i = 0; i < mb; ++i) mem |= (uint64_t)mrow[m0 + i] << (8 * i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < mb; ++i) mem |= (uint64_t)(m0 + i < mend ? mrow[m0 + i] : 0) << (8 * i);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const uint32_t m = mb > 0 ? (uint32_t)(mem >> (j * mb)) & ((1u << mb) - 1u) : 0u;
+    level[j] = (m << 2) | (((e1 >> (8 + j)) & 1u) << 1) | ((e0 >> (8 + j)) & 1u);
   }
 }
 
-__global__ void decode_rows_kernel(DecodeArgs a, const uint16_t* __restrict__ scales,
-                                   const uint16_t* __restrict__ codebook,
-                                   uint16_t* __restrict__ out, int64_t out_stride) {
-  const int64_t r = blockIdx.y;
+// Decode kernels: a thread per 8 columns, a workgroup along the columns and
+// then the rows; 8 weights (16 bytes) or levels (8 bytes) per store where rows
+// are aligned for it.  Bound by issue and the output's write: 2560 x 9728,
+// k=3, weights 19.7 us (2.5 TB/s written; one thread per weight, each with its
+// own byte-wise field reads and 2-byte store: 113.5 us; 1024 x 1024 6.9 -> 3.5 us).
+template <int BITS>
+__global__ void __launch_bounds__(256)
+window_decode_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, uint8_t* __restrict__ out, int64_t out_stride,
+                     bool wide) {
+  const int64_t r = (int64_t)blockIdx.y * blockDim.y + threadIdx.y;
+  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (r >= a.n_rows || c >= a.d) return;
+  uint32_t level[8];
+  levels_of_8<BITS>(a, dm0, dm1, r, c, level);
+  uint8_t* o = out + r * out_stride + c;
+  if (wide && c + 8 <= a.d) {
+    uint2 w = {0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w.x |= level[j] << (8 * j);
+      w.y |= level[4 + j] << (8 * j);
+    }
+    *reinterpret_cast<uint2*>(o) = w;
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (c + j < a.d) o[j] = (uint8_t)level[j];
+  }
+}
+
+template <int BITS>
+__global__ void __launch_bounds__(256)
+decode_rows_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __restrict__ scales,
+                   const uint16_t* __restrict__ codebook, uint16_t* __restrict__ out, int64_t out_stride,
+                   bool wide) {
+  __shared__ float cb[256];
+  for (int i = threadIdx.y * blockDim.x + threadIdx.x; i < 2 << BITS; i += 256) cb[i] = h2f(codebook[i]);
+  __syncthreads();
+  const int64_t r = (int64_t)blockIdx.y * blockDim.y + threadIdx.y;
+  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (r >= a.n_rows || c >= a.d) return;
+  uint32_t level[8];
+  levels_of_8<BITS>(a, dm0, dm1, r, c, level);
   const float sc = h2f(scales[r]);
-  for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < a.d;
-       c += (int64_t)gridDim.x * blockDim.x) {
-    // fp32 product of two fp16 values is exact; one rounding to fp16.
-    out[r * out_stride + c] = f2h(h2f(codebook[level_at(a, r, c)]) * sc);
+  // fp32 product of two fp16 values is exact; one rounding to fp16.
+  uint32_t w[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    w[j] = (uint32_t)f2h(cb[level[2 * j]] * sc) | ((uint32_t)f2h(cb[level[2 * j + 1]] * sc) << 16);
+  uint16_t* o = out + r * out_stride + c;
+  if (wide && c + 8 <= a.d) {
+    *reinterpret_cast<uint4*>(o) = uint4{w[0], w[1], w[2], w[3]};
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (c + j < a.d) o[j] = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
   }
 }
 
@@ -130,10 +208,23 @@ inline int make_decode_args(const uint8_t* path, int64_t path_stride, const uint
   return TP_OK;
 }
 
-inline dim3 decode_grid(int64_t n_rows, int64_t d) {
-  int64_t bx = (d + 255) / 256;
-  if (bx > 64) bx = 64;
-  return dim3((unsigned)bx, (unsigned)n_rows);
+// Bit t of the result: the subset bit of window generator gw takes the path
+// bit t columns back (window bit m - t).
+inline uint32_t window_delays(uint32_t gw, int m) {
+  uint32_t dm = 0;
+  for (int t = 0; t <= m; ++t) dm |= ((gw >> (m - t)) & 1u) << t;
+  return dm;
+}
+
+// 256 threads over (groups of 8 columns, rows): as many along the columns as
+// a row fills, up to a wave (512 columns).
+inline dim3 decode_block(int64_t d) {
+  unsigned x = 8;
+  while (x < 64 && x * 8 < d) x *= 2;
+  return dim3(x, 256 / x);
+}
+inline dim3 decode_grid(int64_t n_rows, int64_t d, dim3 block) {
+  return dim3((unsigned)((d + 8 * block.x - 1) / (8 * block.x)), (unsigned)((n_rows + block.y - 1) / block.y));
 }
 
 }  // namespace tp
@@ -150,8 +241,14 @@ extern "C" int tp_window_decode_levels(const uint8_t* path, int64_t path_stride,
   if (out_stride < d) return TP_ERR_BAD_DIMS;
   if (n_rows == 0) return TP_OK;
   if (n_rows > 65535) return TP_ERR_BAD_DIMS;
-  hipLaunchKernelGGL(window_decode_kernel, decode_grid(n_rows, d), dim3(256), 0,
-                     (hipStream_t)stream, a, levels_out, out_stride);
+  const bool wide = (((uintptr_t)levels_out | (uintptr_t)out_stride) & 7) == 0;
+  const dim3 block = decode_block(d);
+  using Kernel = decltype(&window_decode_kernel<1>);
+  static constexpr Kernel kernels[7] = {window_decode_kernel<1>, window_decode_kernel<2>, window_decode_kernel<3>,
+                                        window_decode_kernel<4>, window_decode_kernel<5>, window_decode_kernel<6>,
+                                        window_decode_kernel<7>};
+  hipLaunchKernelGGL(kernels[bits - 1], decode_grid(n_rows, d, block), block, 0, (hipStream_t)stream, a,
+                     window_delays(a.g0w, a.m), window_delays(a.g1w, a.m), levels_out, out_stride, wide);
   return launch_status();
 }
 
@@ -168,8 +265,14 @@ extern "C" int tp_decode_rows(const uint8_t* path, int64_t path_stride,
   if (out_stride < d) return TP_ERR_BAD_DIMS;
   if (n_rows == 0) return TP_OK;
   if (n_rows > 65535) return TP_ERR_BAD_DIMS;
-  hipLaunchKernelGGL(decode_rows_kernel, decode_grid(n_rows, d), dim3(256), 0,
-                     (hipStream_t)stream, a, scales, codebook, w_out, out_stride);
+  const bool wide = (((uintptr_t)w_out | (uintptr_t)out_stride * 2) & 15) == 0;
+  const dim3 block = decode_block(d);
+  using Kernel = decltype(&decode_rows_kernel<1>);
+  static constexpr Kernel kernels[7] = {decode_rows_kernel<1>, decode_rows_kernel<2>, decode_rows_kernel<3>,
+                                        decode_rows_kernel<4>, decode_rows_kernel<5>, decode_rows_kernel<6>,
+                                        decode_rows_kernel<7>};
+  hipLaunchKernelGGL(kernels[bits - 1], decode_grid(n_rows, d, block), block, 0, (hipStream_t)stream, a,
+                     window_delays(a.g0w, a.m), window_delays(a.g1w, a.m), scales, codebook, w_out, out_stride, wide);
   return launch_status();
 }
 
