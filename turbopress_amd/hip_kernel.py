@@ -318,10 +318,11 @@ def forward_tiled(layer, x: Tensor) -> Tensor:
     _require_cuda(x, "x")
     n, d = layer.out_features, layer.in_features
     flat = x.reshape(-1, d).to(torch.float16).contiguous()
-    y = torch.empty(flat.shape[0], n, dtype=torch.float16, device=x.device)
-    if flat.shape[0] > 32 and forward_prefill(layer, flat, y, layer.bias):
+    rows = flat.shape[0]
+    y = torch.empty(rows, n, dtype=torch.float16, device=x.device)
+    if rows > 32 and forward_prefill(layer, flat, y, layer.bias):
         return y.reshape(*x.shape[:-1], n)
-    if d % 4 or (flat.shape[0] > 8 and (layer.block > 512 or d % 8)):
+    if d % 4 or (rows > 8 and (layer.block > 512 or d % 8)):
         # Rows not 8-byte aligned, or a batch whose Hadamard blocks span more
         # than one 512-column chunk: rotate into the padded layout, then GEMV.
         zpad = rotate_padded(flat, layer.rot_scale, layer.block, layer._tiled_geo["z_cols"])
@@ -332,8 +333,8 @@ def forward_tiled(layer, x: Tensor) -> Tensor:
     bias = layer.bias
     stream = current_stream_ptr(x.device)
     lib = _lib.lib()
-    for b0 in range(0, flat.shape[0], 32):
-        nb = min(32, flat.shape[0] - b0)
+    for b0 in range(0, rows, 32):
+        nb = min(32, rows - b0)
         ws, ws_bytes = layer_workspace(layer, nb)
         st = lib.tp_packed_linear_forward(
             flat.data_ptr() + 2 * b0 * d, d, nb, layer.rot_scale.data_ptr(), layer.block,
