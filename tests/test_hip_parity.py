@@ -76,6 +76,29 @@ def test_rotated_rows_match_oracle(cuda, rows, d, block, ldz, post):
     assert np.array_equal(out.cpu().numpy().view(np.uint16), ref.astype(np.float16).view(np.uint16))
 
 
+@pytest.mark.parametrize("bits", [1, 2, 3, 4, 6])
+@pytest.mark.parametrize("n,d,batch", [(1, 8, 1), (130, 1032, 4), (1500, 576, 16), (1500, 576, 17), (33, 3000, 7)])
+def test_tiled_mode_matches_oracle(cuda, bits, n, d, batch):
+    """mode "tiled" on both sides of its row bound (one GEMV launch / decoded
+    row tiles), with bias, against the fp64 product of the exact weights
+    codebook * scale and activations.  Each fp16 rounding is at most 2^-11 of
+    its value: z and (row tiles) w once per term, the product and the sum with
+    the bias once, so |y - ref| <= 2^-11 (4 sum |w z| + 2 |bias|), where the
+    rotated z's own rounding is at most 2^-11 |z|."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    p = make_payload(n, d, bits, 16, seed=n + d, bias=True)
+    lin = PackedTCQLinear(p, mode="tiled", tile_rows=512)
+    x = make_activation(batch, d, seed=batch)
+    y = lin(x.to(cuda)).double().cpu().numpy()
+    pn = payload_numpy(p)
+    w = pn["codebook"].astype(np.float64)[O.levels_of(pn)] * pn["scales"].astype(np.float64)[:, None]
+    rs = O.rot_scale(pn["signs_packed"], pn["inv_equil"], d).astype(np.float64)
+    z = O.block_fwht(x.numpy().astype(np.float64) * rs, p["block"])
+    ref = z @ w.T + pn["bias"].astype(np.float64)
+    bound = 2.0 ** -11 * (4 * (np.abs(z) @ np.abs(w).T) + 2 * np.abs(pn["bias"].astype(np.float64)))
+    assert np.all(np.abs(y - ref) <= bound)
+
+
 def test_fwht_scale_rejects_bad_block(cuda):
     from turbopress_amd.hip_kernel import fwht_scale
     x = torch.zeros(1, 96, dtype=torch.float16, device=cuda)
@@ -150,6 +173,11 @@ GEMV_CASES = [
     (64, 128, 1, 4, 1),
     (96, 320, 5, 64, 9),
 ]
+# the natural-stream GEMV's edges: 1, 4 and 8 rows at once and remainders, one
+# wave per row and four, rows of no multiple of 8 columns, more columns than
+# one span of four waves
+GEMV_CASES += [(n, d, k, 64, b) for k in (1, 5, 6, 7) for n, d, b in
+               ((1, 1, 1), (5, 515, 3), (66, 1032, 5), (7, 1100, 8), (3, 4104, 17), (4100, 1536, 2))]
 
 
 @pytest.mark.parametrize("n,d,bits,n_states,batch", GEMV_CASES)

@@ -58,35 +58,6 @@ inline int trellis_taps(int n_states, TrellisTaps* t) {
   return TP_OK;
 }
 
-__device__ __forceinline__ uint32_t subset_of_window(uint32_t x, uint32_t g0w, uint32_t g1w) {
-  return ((__popc(x & g1w) & 1u) << 1) | (__popc(x & g0w) & 1u);
-}
-
-// Little-endian bit-field read of `width` (<= 25) bits starting at stream bit
-// `bit` of a byte row; bytes at or beyond `row_bytes` read as zero.
-__device__ __forceinline__ uint32_t read_bits_le(const uint8_t* row, int64_t row_bytes,
-                                                 int64_t bit, int width) {
-  int64_t byte0 = bit >> 3;
-  uint32_t v = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int64_t b = byte0 + i;
-    uint32_t byte = (b < row_bytes) ? (uint32_t)row[b] : 0u;
-    v |= byte << (8 * i);
-  }
-  return (v >> (bit & 7)) & ((1u << width) - 1u);
-}
-
-// Path window of weight t in a row: bits b[t-m .. t], zero before the row.
-__device__ __forceinline__ uint32_t path_window(const uint8_t* row, int64_t row_bytes,
-                                                int64_t t, int m) {
-  int64_t lo = t - m;
-  if (lo >= 0) return read_bits_le(row, row_bytes, lo, m + 1);
-  // Row start: only bits 0..t exist; they land at window bits (m-t)..m.
-  uint32_t v = read_bits_le(row, row_bytes, 0, (int)(t + 1));
-  return v << (uint32_t)(-lo);
-}
-
 __device__ __forceinline__ float h2f(uint16_t h) {
   return __half2float(__ushort_as_half(h));
 }

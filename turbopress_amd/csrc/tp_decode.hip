@@ -28,18 +28,6 @@ struct DecodeArgs {
   uint32_t g0w, g1w;
 };
 
-__device__ __forceinline__ uint32_t level_at(const DecodeArgs& a, int64_t r, int64_t c) {
-  const uint8_t* prow = a.path + r * a.path_stride;
-  uint32_t win = path_window(prow, a.path_stride, c, a.m);
-  uint32_t sub = subset_of_window(win, a.g0w, a.g1w);
-  uint32_t mem = 0;
-  if (a.bits > 1) {
-    const uint8_t* mrow = a.member + r * a.member_stride;
-    mem = read_bits_le(mrow, a.member_stride, c * (a.bits - 1), a.bits - 1);
-  }
-  return mem * 4u + sub;
-}
-
 // The 8 columns from c (a multiple of 8) of row r: their path bits are byte
 // c / 8 of the row, the up to 6 bits before them the byte before it (zero at
 // the row's start), their members the bits - 1 bytes from c / 8 * (bits - 1)
@@ -138,47 +126,110 @@ decode_rows_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __r
   }
 }
 
-// One wave per output row; lanes stride over the columns; the batch is
-// processed in chunks of 8 accumulators.
-constexpr int kGenericBatchChunk = 8;
-
+// GEMV on the natural streams: WPR waves of a workgroup share an output row, a
+// lane takes 8 columns at a time (levels_of_8, one 16-byte read of z per batch
+// row) for NB batch rows at once; sums over lanes, then over the waves of a
+// row through LDS, in a fixed order.  WIDE: rows of z are whole 16-byte groups.
+// Bound by issue (decode and conversions, ~15 instructions per weight and lane
+// at 4 batch rows) on large linears and by one or two load round trips on
+// small ones: at 1 / 4 / 8 batch rows 9728 x 2560 (k=4) 13.3 / 16.1 / 20.9 us,
+// 3072 x 1024 (k=3) 5.2 / 6.8 / 9.9 us.  (A thread per weight, fields read byte
+// by byte: k=4 gate_proj at batch 1 127 us.)
+template <int BITS, int NB, int WPR, bool WIDE>
 __global__ void __launch_bounds__(256)
-generic_gemv_kernel(DecodeArgs a, const uint16_t* __restrict__ z, int64_t batch,
+generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __restrict__ z, int nb,
                     const uint16_t* __restrict__ scales, const uint16_t* __restrict__ codebook,
                     const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t n) {
-  __shared__ float cb[256];
-  const int ncb = 1 << (a.bits + 1);
-  for (int i = threadIdx.x; i < ncb; i += blockDim.x) cb[i] = h2f(codebook[i]);
+  __shared__ float cb[2 << BITS];
+  __shared__ float part[4][NB];
+  for (int i = threadIdx.x; i < 2 << BITS; i += 256) cb[i] = h2f(codebook[i]);
   __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-  if (r >= n) return;
-  const float sc = h2f(scales[r]);
-  for (int64_t b0 = 0; b0 < batch; b0 += kGenericBatchChunk) {
-    const int nb = (int)((batch - b0) < kGenericBatchChunk ? (batch - b0) : kGenericBatchChunk);
-    float acc[kGenericBatchChunk];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t r = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
+  const int64_t rr = r < n ? r : n - 1;  // (waves past the last row repeat it and write nothing)
+  float acc[NB];
 #pragma unroll
-    for (int b = 0; b < kGenericBatchChunk; ++b) acc[b] = 0.f;
-    for (int64_t c = lane; c < a.d; c += 64) {
-      const float w = cb[level_at(a, r, c)];
+  for (int b = 0; b < NB; ++b) acc[b] = 0.f;
+  for (int64_t c = (int64_t)(wave % WPR) * 512 + lane * 8; c < a.d; c += 512 * WPR) {
+    uint4 zw[NB];
 #pragma unroll
-      for (int b = 0; b < kGenericBatchChunk; ++b)
-        if (b < nb) acc[b] += w * h2f(z[(b0 + b) * a.d + c]);
-    }
+    for (int b = 0; b < NB; ++b) {
+      const uint16_t* zb = z + (b < nb ? b : 0) * a.d + c;  // (batch rows past nb: row 0, not written)
+      if constexpr (WIDE) {
+        zw[b] = *reinterpret_cast<const uint4*>(zb);
+      } else {
+        uint32_t e[8];
 #pragma unroll
-    for (int b = 0; b < kGenericBatchChunk; ++b) {
-      float v = acc[b];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-      acc[b] = v;
-    }
-    if (lane == 0) {
-      for (int b = 0; b < nb; ++b) {
-        uint16_t out = f2h(acc[b] * sc);
-        if (bias) out = f2h(h2f(out) + h2f(bias[r]));
-        y[(b0 + b) * n + r] = out;
+        for (int j = 0; j < 8; ++j) e[j] = c + j < a.d ? zb[j] : 0;
+        zw[b] = uint4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
       }
     }
+    uint32_t level[8];
+    levels_of_8<BITS>(a, dm0, dm1, rr, c, level);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float w = cb[level[j]];
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        const uint32_t zz = j < 2 ? zw[b].x : j < 4 ? zw[b].y : j < 6 ? zw[b].z : zw[b].w;
+        acc[b] += w * h2f((uint16_t)(zz >> (16 * (j & 1))));
+      }
+    }
+  }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) acc[b] += __shfl_xor(acc[b], off, 64);
+  }
+  if constexpr (WPR > 1) {
+    if (lane == 0) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) part[wave][b] = acc[b];
+    }
+    __syncthreads();
+    if (wave % WPR) return;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int w = 1; w < WPR; ++w) acc[b] += part[wave + w][b];
+  }
+  if (lane == 0 && r < n) {
+    const float sc = h2f(scales[r]);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      if (b >= nb) continue;
+      uint16_t out = f2h(acc[b] * sc);
+      if (bias) out = f2h(h2f(out) + h2f(bias[r]));
+      y[b * n + r] = out;
+    }
+  }
+}
+
+template <int BITS, int NB>
+void launch_generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* z, int nb,
+                         const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias, uint16_t* y,
+                         int64_t n, hipStream_t s) {
+  const bool wide = (a.d & 7) == 0 && ((uintptr_t)z & 15) == 0;
+  // four waves per row while a wave per row leaves CUs short of waves
+  const bool split = a.d > 1024 && n < (int64_t)16 * device_cu_count();
+  auto kern = split ? (wide ? generic_gemv_kernel<BITS, NB, 4, true> : generic_gemv_kernel<BITS, NB, 4, false>)
+                    : (wide ? generic_gemv_kernel<BITS, NB, 1, true> : generic_gemv_kernel<BITS, NB, 1, false>);
+  const int64_t rows = split ? 1 : 4;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((n + rows - 1) / rows)), dim3(256), 0, s, a, dm0, dm1, z, nb, scales,
+                     codebook, bias, y, n);
+}
+
+template <int BITS>
+void generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* z, int64_t batch,
+                  const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias, uint16_t* y, int64_t n,
+                  hipStream_t s) {
+  for (int64_t b0 = 0; b0 < batch; b0 += 8) {
+    const int nb = (int)(batch - b0 < 8 ? batch - b0 : 8);
+    const uint16_t* zb = z + b0 * a.d;
+    uint16_t* yb = y + b0 * n;
+    if (nb == 1) launch_generic_gemv<BITS, 1>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
+    else if (nb <= 4) launch_generic_gemv<BITS, 4>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
+    else launch_generic_gemv<BITS, 8>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
   }
 }
 
@@ -289,9 +340,10 @@ extern "C" int tp_tcq_gemv(const uint16_t* z, int64_t batch,
   if (!z || !scales || !codebook || !y) return TP_ERR_NULL_POINTER;
   if (batch < 0) return TP_ERR_BAD_DIMS;
   if (batch == 0 || n == 0) return TP_OK;
-  const int rows_per_block = 4;
-  dim3 grid((unsigned)((n + rows_per_block - 1) / rows_per_block));
-  hipLaunchKernelGGL(generic_gemv_kernel, grid, dim3(64 * rows_per_block), 0,
-                     (hipStream_t)stream, a, z, batch, scales, codebook, bias, y, n);
+  const uint32_t dm0 = window_delays(a.g0w, a.m), dm1 = window_delays(a.g1w, a.m);
+  using Gemv = decltype(&generic_gemv<1>);
+  static constexpr Gemv gemv[7] = {generic_gemv<1>, generic_gemv<2>, generic_gemv<3>, generic_gemv<4>,
+                                   generic_gemv<5>, generic_gemv<6>, generic_gemv<7>};
+  gemv[bits - 1](a, dm0, dm1, z, batch, scales, codebook, bias, y, n, (hipStream_t)stream);
   return launch_status();
 }

@@ -35,6 +35,13 @@ __all__ = ["PackedTCQLinear", "MODES", "Trellis", "trellis_generators", "pack_li
 
 MODES = ("hip", "triton", "cached", "tiled")
 
+# Rows up to which mode "tiled" multiplies straight from the packed streams
+# (one launch, weights unrounded) instead of decoding row tiles: one pass of
+# the natural-stream GEMV per 8 rows.  16 rows: 9728 x 2560 48 us (row tiles
+# 396), 4096 x 9728, k=4, 71 us (168); at 32 rows of the latter 136 us, which a
+# larger tile_rows than the default 1024 can beat.
+_TILED_GEMV_ROWS = 16
+
 _GENERATORS = {4: (0o5, 0o7), 8: (0o15, 0o17), 16: (0o23, 0o35), 64: (0o133, 0o171)}
 
 
@@ -210,7 +217,7 @@ class PackedTCQLinear(nn.Module):
         if self.tiled_packed is not None:
             return hk.forward_tiled(self, x).to(x.dtype)
         z = hk.fwht_scale(x, self.rot_scale, self.block)
-        if self._packed_path:
+        if self._packed_path or z.numel() <= _TILED_GEMV_ROWS * self.in_features:
             y = hk.packed_gemv(z, self, bias=self.bias)
         else:  # tiled
             flat = z.reshape(-1, self.in_features)
