@@ -230,6 +230,32 @@ def test_prompt_forward_matches_oracle_deterministically(cuda, n, d, bits, n_sta
     assert torch.equal(out, y) and bool((guard[batch * n:] == 7.0).all())
 
 
+def test_prompt_forward_in_pieces(cuda, monkeypatch):
+    """More rows than one prompt GEMM takes: whole pieces and a shorter last
+    one (with a plan, and K parts, of its own) match the call in one piece."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    p = make_payload(700, 2560, 3, 64, seed=5, bias=True)
+    lin = PackedTCQLinear(p, mode="hip")
+    x = make_activation(300, 2560, seed=6).to(cuda)
+    whole = lin(x).float()
+    monkeypatch.setattr(hk, "_PREFILL_ROWS", 128)
+    pieces = lin(x).float()
+    # (other K parts add the same fp32 products in another order: one fp16 ulp)
+    assert float((pieces - whole).abs().max()) <= 2.0 ** -10 * float(whole.abs().max())
+
+
+@pytest.mark.parametrize("n,d,bits,batch", [(512, 1024, 2, 17), (511, 1024, 2, 17), (600, 4096, 3, 31), (1000, 2560, 4, 32),
+                                            (513, 1030, 3, 24), (3449, 9728, 3, 17), (3450, 9728, 2, 32)])
+def test_forward_of_17_to_32_rows(cuda, n, d, bits, batch):
+    """17..32 rows on both sides of the sizes that take the prompt GEMM."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    p = make_payload(n, d, bits, 64, seed=n + d, bias=True)
+    lin = PackedTCQLinear(p, mode="hip")
+    x = make_activation(batch, d, seed=batch)
+    y = lin(x.to(cuda)).float().cpu().numpy()
+    assert O.max_rel(y, O.tiled_forward(payload_numpy(p), x.numpy())) <= GEMV_TOL
+
+
 def test_fused_equals_two_launch_path(cuda):
     from turbopress_amd import hip_kernel as hk
     from turbopress_amd.runtime import PackedTCQLinear

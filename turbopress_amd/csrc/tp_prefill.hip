@@ -176,6 +176,9 @@ tcq_prefill_kernel(const PrefillArgs a) {
   const int h = lane >> 5, r = lane & 15, tsel = (lane >> 4) & 1;
   const uint32_t laneoff = lane_offsets<KB>(lane);
 
+  // (first of the loads: the table is built while the others are in flight)
+  const uint32_t cb_lane = gld(a.codebook + (lane & ((2 << KB) - 1)));
+
   // tile of this workgroup: each XCD (blockIdx % 8) takes a contiguous run
   const int total = (int)gridDim.x, q8 = total >> 3, r8 = total & 7;
   const int xcd = (int)blockIdx.x & 7;
@@ -241,7 +244,7 @@ tcq_prefill_kernel(const PrefillArgs a) {
     if (a.bias) brow = gld(a.bias + erow);
   }
 
-  build_pair_table_lanes<KB>(table, (uint32_t)a.codebook[lane & ((2 << KB) - 1)], tid, 128 * WM);
+  build_pair_table_lanes<KB>(table, cb_lane, tid, 128 * WM);
 
   float16_t acc[MG][NG];
 #pragma unroll

@@ -282,36 +282,40 @@ _PREFILL_ROWS = 32768  # rows per prompt GEMM (bounds its workspace)
 
 
 def forward_prefill(layer, flat: Tensor, y: Tensor, bias: Tensor | None, rotated: bool = False) -> bool:
-    """y = forward of more than 32 rows `flat` (contiguous fp16 [B, d]; with
+    """y = forward of many rows `flat` (contiguous fp16 [B, d]; with
     `rotated` they are z already) by the prompt GEMM (tp_packed_linear_prefill);
     False for sizes it does not take."""
     n, d = layer.out_features, layer.in_features
     rot, block = (0, 1) if rotated else (layer.rot_scale.data_ptr(), layer.block)
     lib = _lib.lib()
     rows = flat.shape[0]
-    need = int(lib.tp_prefill_workspace_bytes(n, d, min(rows, _PREFILL_ROWS), layer.bits))
+    nb = rows if rows <= _PREFILL_ROWS else _PREFILL_ROWS
+    need = lib.tp_prefill_workspace_bytes(n, d, nb, layer.bits)
     if need <= 0:
         return False
-    ws = None
-    buf = layer.tiled_packed
+    ws = torch.empty(need, dtype=torch.uint8, device=flat.device)
+    path = layer.tiled_packed.data_ptr()
+    member = path + layer._tiled_geo["path_bytes"]
+    scales, codebook = layer.scales.data_ptr(), layer.codebook.data_ptr()
+    bias_ptr = 0 if bias is None else bias.data_ptr()
+    xp, yp = flat.data_ptr(), y.data_ptr()
     stream = current_stream_ptr(flat.device)
     for b0 in range(0, rows, _PREFILL_ROWS):
-        nb = min(_PREFILL_ROWS, rows - b0)
-        need = int(lib.tp_prefill_workspace_bytes(n, d, nb, layer.bits))
-        if ws is None or ws.numel() < need:
-            ws = torch.empty(need, dtype=torch.uint8, device=flat.device)
-        st = lib.tp_packed_linear_prefill(
-            flat.data_ptr() + 2 * b0 * d, nb, rot, block, buf.data_ptr(),
-            buf.data_ptr() + layer._tiled_geo["path_bytes"], layer.scales.data_ptr(),
-            layer.codebook.data_ptr(), 0 if bias is None else bias.data_ptr(), n, d, layer.bits,
-            layer.n_states, y.data_ptr() + 2 * b0 * n, n, ws.data_ptr(), ws.numel(), stream)
+        if rows - b0 < nb:  # a shorter last piece has a plan of its own
+            nb = rows - b0
+            need = lib.tp_prefill_workspace_bytes(n, d, nb, layer.bits)
+            if ws.numel() < need:
+                ws = torch.empty(need, dtype=torch.uint8, device=flat.device)
+        st = lib.tp_packed_linear_prefill(xp + 2 * b0 * d, nb, rot, block, path, member, scales, codebook, bias_ptr,
+                                          n, d, layer.bits, layer.n_states, yp + 2 * b0 * n, n, ws.data_ptr(),
+                                          ws.numel(), stream)
         _lib.check(st, "packed_linear_prefill")
     return True
 
 
 def forward_tiled(layer, x: Tensor) -> Tensor:
-    """Rotation + decode-GEMV + bias: more than 32 rows run the prompt GEMM
-    (forward_prefill); up to 32 one fused launch (tp_packed_linear_forward)
+    """Rotation + decode-GEMV + bias: more than 16 rows run the prompt GEMM
+    (forward_prefill); fewer one fused launch (tp_packed_linear_forward)
     when the rotation fits the launch (up to 8 rows, or Hadamard blocks <=
     512), otherwise the rows rotate once into the padded layout and run the
     batched decode-GEMV (tp_tcq_gemv_tiled).  fp16 [..., n]."""
@@ -320,7 +324,16 @@ def forward_tiled(layer, x: Tensor) -> Tensor:
     flat = x.reshape(-1, d).to(torch.float16).contiguous()
     rows = flat.shape[0]
     y = torch.empty(rows, n, dtype=torch.float16, device=x.device)
-    if rows > 32 and forward_prefill(layer, flat, y, layer.bias):
+    # 17..32 rows too where the fused launch does not rotate (Hadamard blocks
+    # above 512) or decodes 2^25 weights or more: 32 rows of 2560 x 4096 (block
+    # 4096) 19.5 -> 15.9 us of GPU time and 32.2 -> 23.5 us per eager call, 4096
+    # x 9728 27.5 -> 23.0 per call.  Below that the one launch is cheaper to call
+    # (9728 x 2560 20.6 against 23.5 us, though 20.6 against 16.6 of GPU time),
+    # with few rows of weights K parts leave the GEMM short of workgroups (300 x
+    # 9216: 15.4 against 17.7), and 9..16 rows fill half of its columns (16 rows
+    # of 2560 x 4096: 15.1 against 15.7).
+    if rows > 16 and (rows > 32 or n >= 512 and (layer.block > 512 or n * d >= 1 << 25)) \
+            and forward_prefill(layer, flat, y, layer.bias):
         return y.reshape(*x.shape[:-1], n)
     if d % 4 or (rows > 8 and (layer.block > 512 or d % 8)):
         # Rows not 8-byte aligned, or a batch whose Hadamard blocks span more
