@@ -176,6 +176,18 @@ static void argument_cases() {
     EXPECT(tp_packed_linear_forward(h, 1024, 6, h, 1024, b, b, h, h, nullptr, n, 1024, 3, 64, o, n, ws, need - 4,
                                     nullptr) == TP_ERR_WORKSPACE);
   }
+  EXPECT(tp_prefill_workspace_bytes(1 << 20, 256, 65536, 3) == 0);
+  EXPECT(tp_prefill_workspace_bytes(33, INT64_MAX, 33, 3) == 0);
+  for (int64_t batch : {33, 199, 2048, 65535})
+    for (int64_t n : {33, 2560, 9728}) EXPECT(tp_prefill_workspace_bytes(n, 9728, batch, 3) >= batch * 9728 * 2);
+  EXPECT(tp_packed_linear_prefill(nullptr, 64, h, 256, b, b, h, h, nullptr, 16, 256, 3, 64, o, 16, o, 1 << 20,
+                                  nullptr) == TP_ERR_NULL_POINTER);
+  EXPECT(tp_packed_linear_prefill(h, 64, h, 256, b, b, h, h, nullptr, 16, 256, 9, 64, o, 16, o, 1 << 20, nullptr) ==
+         TP_ERR_UNSUPPORTED_BITS);
+  EXPECT(tp_packed_linear_prefill(h, 64, h, 256, b, b, h, h, nullptr, 16, 256, 3, 64, o, 16, o,
+                                  tp_prefill_workspace_bytes(16, 256, 64, 3) - 16, nullptr) == TP_ERR_WORKSPACE);
+  EXPECT(tp_packed_linear_prefill(h, 64, h, 256, b, b, h, h, nullptr, 16, 256, 3, 64, o, 15, o, 1 << 20, nullptr) ==
+         TP_ERR_BAD_DIMS);
   EXPECT(tp_tcq_viterbi(nullptr, 256, 16, 256, nullptr, 3, 64, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                         0, nullptr) != TP_OK);
   EXPECT(tp_read_probe(nullptr, 64, nullptr, nullptr) != TP_OK);

@@ -499,10 +499,8 @@ int64_t pre_workspace(const PrePlan& p, int64_t U) {
 // Sizes the kernel's 32-bit offsets and grid hold (a column group of z below
 // 2^31 bytes); rows: what one rotation launch takes.
 int pre_geom(int64_t n, int64_t d, int64_t batch, int bits, Geom* g) {
-  const int st = tiled_geom(n, d, bits, g);
-  if (st) return st;
-  if (batch < 1 || batch > 65535 || g->G4 > 4096 || n > (1 << 24)) return TP_ERR_BAD_DIMS;
-  return TP_OK;
+  if (batch < 1 || batch > 65535 || d > (1 << 20) || n > (1 << 24)) return TP_ERR_BAD_DIMS;
+  return tiled_geom(n, d, bits, g);
 }
 
 }  // namespace
