@@ -4,7 +4,7 @@ the per-row quantizer around it (``trellis.py:256-320``).
 
 ``viterbi`` returns exactly what the reference's ``_viterbi`` returns --
 ``(level_codes, path_bits, member_codes, end_state)`` -- computed by
-``tp_tcq_viterbi`` (one wave per row, one lane per trellis state; see
+``tp_tcq_viterbi`` (one wave per row, the trellis in place across its lanes; see
 ``csrc/tp_viterbi.hip``) with the reference's fp32 arithmetic and
 tie-breaking, so the codes are identical.  Rows are processed in chunks so
 the branch-decision workspace (8 bytes per weight) stays bounded.
