@@ -20,13 +20,16 @@
 // each of them: 1316 us for 2048 rows of a 9728 x 2560 linear (k=3) and 122 us
 // for 199 rows of 2560 x 4096, against 128 and 25 us here.
 //
-// What bounds the GEMM: at 2048 x 2560 x 9728 the launch takes 115-130 us
-// (0.79-0.89 PFLOP/s; a dense fp16 library product of that shape 103-117 us on
-// the same card).  In its main loop the matrix cores are ~75-80 % busy at the
-// 1.6-1.7 GHz the power limit leaves this load, LDS ~70 % (pair lookups: 4
-// reads of 4 bytes per lane and A operand; batch operands: one 16-byte read
-// per MG MFMAs), VALU ~40 %.  Decode cost per MFMA falls with NG, batch reads
-// with MG; 2 waves per SIMD hide both behind the other wave's MFMAs.
+// What bounds the GEMM: at 2048 x 2560 x 9728 the launch takes 112-130 us
+// (0.79-0.91 PFLOP/s; a dense fp16 library product of that shape 103-117 us on
+// the same card).  While workgroups are resident the matrix cores are busy 61 %
+// of the SIMD cycles (128 x 256 tiles; 70 % with 256 x 256 ones, which fill
+// fewer CUs here) at the 1.7-1.8 GHz that the power limit leaves, LDS 50 % (pair
+// lookups: 4 reads of 4 bytes per lane and A operand; batch operands: one
+// 16-byte read per MG MFMAs), other vector instructions 33 %; the rest is each
+// tile's table, first loads and output, and the last of 2.4 passes over the
+// CUs.  Decode cost per MFMA falls with NG, batch reads with MG; 2 waves per
+// SIMD hide both behind the other wave's MFMAs.
 #include "tp_slot.h"
 
 #include <algorithm>

@@ -25,7 +25,7 @@
 // read (v_readlane) per column, collecting the lane sequence 32 columns at a
 // time into one register (a lane per column); the lanes then emit path bit,
 // subset, member and level of their columns in parallel.
-// Bound by instruction issue (VALU), 9728 rows x 2560 columns, k=3, S=64:
+// Bound by VALU issue (96 % of the SIMD cycles), 9728 x 2560, k=3, S=64:
 // 577 us per search.  (With lane = state, both subset costs computed in every
 // lane and two LDS shuffles per column: 1470 us; 2560 x 2560, k=2, S=4: 486 us,
 // here 205.)
