@@ -192,6 +192,29 @@ def test_packed_gemv_matches_fp64_oracle(cuda, n, d, bits, n_states, batch):
     assert O.max_rel(y, ref) <= GEMV_TOL
 
 
+@pytest.mark.parametrize("mode,bits", [("tiled", 2), ("tiled", 4), ("hip", 5), ("hip", 7)])
+@pytest.mark.parametrize("d,batch", [(13, 1), (2051, 4), (1031, 8)])
+def test_unused_infinite_levels_do_not_reach_the_output(cuda, mode, bits, d, batch):
+    """The natural-stream GEMV over rows of no multiple of 8 columns: the
+    stream bits past a row's end decode to levels 0..3, whose entries are
+    infinite or NaN here and which no weight uses (every member code is at
+    least 1); the products must match the fp64 ones of the weights alone."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    n, mb = 5, bits - 1
+    p = make_payload(n, d, bits, 64, seed=d)
+    field = torch.zeros(n, (d * mb + 7) // 8 * 8, dtype=torch.uint8)
+    field[:, :d * mb:mb] = 1  # member code 1 everywhere, zero bits after the row
+    p["member_packed"] = (field.reshape(n, -1, 8) << torch.arange(8, dtype=torch.uint8)).sum(-1).to(torch.uint8)
+    p["codebook"][:4] = torch.tensor([float("inf"), float("-inf"), float("nan"), float("inf")], dtype=torch.float16)
+    lin = PackedTCQLinear(p, mode=mode)
+    x = make_activation(batch, d, seed=batch)
+    y = lin(x.to(cuda)).float().cpu().numpy()
+    pn = payload_numpy(p)
+    rs = O.rot_scale(pn["signs_packed"], pn["inv_equil"], d).astype(np.float32)
+    z = O.block_fwht(x.numpy().astype(np.float32) * rs, p["block"]).astype(np.float16)
+    assert O.max_rel(y, O.gemv_fp64(pn, z.astype(np.float64))) <= GEMV_TOL
+
+
 @pytest.mark.parametrize("mode", ["hip", "triton", "tiled", "cached"])
 @pytest.mark.parametrize("n,d,bits", [(1536, 576, 2), (256, 1024, 3), (72, 640, 4)])
 def test_forward_modes_match_tiled_oracle(cuda, mode, n, d, bits):

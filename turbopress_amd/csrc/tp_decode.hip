@@ -168,7 +168,8 @@ generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __
     levels_of_8<BITS>(a, dm0, dm1, rr, c, level);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float w = cb[level[j]];
+      // (past the row's end z is zero, but a zero times an infinite or NaN entry is not)
+      const float w = WIDE || c + j < a.d ? cb[level[j]] : 0.f;
 #pragma unroll
       for (int b = 0; b < NB; ++b) {
         const uint32_t zz = j < 2 ? zw[b].x : j < 4 ? zw[b].y : j < 6 ? zw[b].z : zw[b].w;
