@@ -192,6 +192,39 @@ def test_packed_gemv_matches_fp64_oracle(cuda, n, d, bits, n_states, batch):
     assert O.max_rel(y, ref) <= GEMV_TOL
 
 
+@pytest.mark.parametrize("n,d,bits,batch", [(16, 64, 5, 33), (192, 256, 1, 199), (70, 1100, 7, 9), (5, 515, 6, 37),
+                                            (33, 1032, 5, 2048), (300, 2056, 5, 44)])
+def test_natural_streams_take_any_rows_in_one_launch(cuda, n, d, bits, batch):
+    """packed_gemv of more than 8 rows at rates without a device layout: last
+    groups of 1, 3, 4, 5 and 8 rows, every row against the fp64 product
+    relative to the row's own largest value, one graph node, replays equal to
+    the eager result."""
+    import ctypes
+    from turbopress_amd import _lib
+    from turbopress_amd.hip_kernel import packed_gemv
+    from turbopress_amd.runtime import PackedTCQLinear
+    p = make_payload(n, d, bits, 64, seed=n + d)
+    lin = PackedTCQLinear(p, mode="hip")
+    z = torch.randn(batch, d, generator=torch.Generator().manual_seed(1)).to(torch.float16)
+    zd = z.to(cuda)
+    y = packed_gemv(zd, lin)
+    ref = O.gemv_fp64(payload_numpy(p), z.numpy().astype(np.float64))
+    err = np.abs(y.double().cpu().numpy() - ref).max(axis=1)
+    assert np.all(err <= GEMV_TOL * np.abs(ref).max(axis=1))
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out = packed_gemv(zd, lin)
+    count = ctypes.c_size_t(0)
+    assert _lib.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(count)) == 0
+    assert count.value == 1
+    graph.instantiate()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, y)
+
+
 @pytest.mark.parametrize("mode,bits", [("tiled", 2), ("tiled", 4), ("hip", 5), ("hip", 7)])
 @pytest.mark.parametrize("d,batch", [(13, 1), (2051, 4), (1031, 8)])
 def test_unused_infinite_levels_do_not_reach_the_output(cuda, mode, bits, d, batch):

@@ -136,14 +136,10 @@ decode_rows_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __r
 // 3072 x 1024 (k=3) 5.2 / 6.8 / 9.9 us.  (A thread per weight, fields read byte
 // by byte: k=4 gate_proj at batch 1 127 us.)
 template <int BITS, int NB, int WPR, bool WIDE>
-__global__ void __launch_bounds__(256)
-generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __restrict__ z, int nb,
-                    const uint16_t* __restrict__ scales, const uint16_t* __restrict__ codebook,
-                    const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t n) {
-  __shared__ float cb[2 << BITS];
-  __shared__ float part[4][NB];
-  for (int i = threadIdx.x; i < 2 << BITS; i += 256) cb[i] = h2f(codebook[i]);
-  __syncthreads();
+__device__ __forceinline__ void
+gemv_batch_rows(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* __restrict__ z, int nb,
+                const uint16_t* __restrict__ scales, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
+                int64_t n, const float* cb, float* part) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t r = (int64_t)blockIdx.x * (4 / WPR) + wave / WPR;
   const int64_t rr = r < n ? r : n - 1;  // (waves past the last row repeat it and write nothing)
@@ -185,14 +181,14 @@ generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __
   if constexpr (WPR > 1) {
     if (lane == 0) {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) part[wave][b] = acc[b];
+      for (int b = 0; b < NB; ++b) part[wave * NB + b] = acc[b];
     }
     __syncthreads();
     if (wave % WPR) return;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int w = 1; w < WPR; ++w) acc[b] += part[wave + w][b];
+      for (int w = 1; w < WPR; ++w) acc[b] += part[(wave + w) * NB + b];
   }
   if (lane == 0 && r < n) {
     const float sc = h2f(scales[r]);
@@ -206,8 +202,37 @@ generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __
   }
 }
 
+// NB = 8: batch rows 8 blockIdx.y on, the last 1..7 of them at their own width;
+// NB = 1, 4: all of them.
+template <int BITS, int NB, int WPR, bool WIDE>
+__global__ void __launch_bounds__(256)
+generic_gemv_kernel(DecodeArgs a, uint32_t dm0, uint32_t dm1, const uint16_t* __restrict__ z, int64_t batch,
+                    const uint16_t* __restrict__ scales, const uint16_t* __restrict__ codebook,
+                    const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t n) {
+  __shared__ float cb[2 << BITS];
+  __shared__ float part[4 * NB];
+  for (int i = threadIdx.x; i < 2 << BITS; i += 256) cb[i] = h2f(codebook[i]);
+  __syncthreads();
+  if constexpr (NB < 8) {
+    gemv_batch_rows<BITS, NB, WPR, WIDE>(a, dm0, dm1, z, (int)batch, scales, bias, y, n, cb, part);
+  } else {
+    const int64_t b0 = (int64_t)blockIdx.y * 8;
+    const int nb = (int)(batch - b0 < 8 ? batch - b0 : 8);
+    z += b0 * a.d;
+    y += b0 * n;
+    if (nb > 4) gemv_batch_rows<BITS, 8, WPR, WIDE>(a, dm0, dm1, z, nb, scales, bias, y, n, cb, part);
+    else if (nb > 1) gemv_batch_rows<BITS, 4, WPR, WIDE>(a, dm0, dm1, z, nb, scales, bias, y, n, cb, part);
+    else gemv_batch_rows<BITS, 1, WPR, WIDE>(a, dm0, dm1, z, nb, scales, bias, y, n, cb, part);
+  }
+}
+
+// One launch for every batch row (65535 groups of 8 at most per launch).  A
+// launch per group of 8 was slower on small linears than the work was: 16 x
+// 64, k=5, 33 rows 37.7 us per eager call with the rotation (here 27.0), 2048
+// rows 1114 (27.2), and every group waited for the one before it: 3072 x 1024,
+// k=5, 64 rows 49 us of GPU time (25.9), 9728 x 2560 at 2048 rows 4924 (3535).
 template <int BITS, int NB>
-void launch_generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* z, int nb,
+void launch_generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* z, int64_t batch,
                          const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias, uint16_t* y,
                          int64_t n, hipStream_t s) {
   const bool wide = (a.d & 7) == 0 && ((uintptr_t)z & 15) == 0;
@@ -216,22 +241,21 @@ void launch_generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const 
   auto kern = split ? (wide ? generic_gemv_kernel<BITS, NB, 4, true> : generic_gemv_kernel<BITS, NB, 4, false>)
                     : (wide ? generic_gemv_kernel<BITS, NB, 1, true> : generic_gemv_kernel<BITS, NB, 1, false>);
   const int64_t rows = split ? 1 : 4;
-  hipLaunchKernelGGL(kern, dim3((unsigned)((n + rows - 1) / rows)), dim3(256), 0, s, a, dm0, dm1, z, nb, scales,
-                     codebook, bias, y, n);
+  const int64_t most = (int64_t)65535 * NB;
+  for (int64_t b0 = 0; b0 < batch; b0 += most) {
+    const int64_t nb = batch - b0 < most ? batch - b0 : most;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + rows - 1) / rows), (unsigned)((nb + NB - 1) / NB)), dim3(256), 0, s, a,
+                       dm0, dm1, z + b0 * a.d, nb, scales, codebook, bias, y + b0 * n, n);
+  }
 }
 
 template <int BITS>
 void generic_gemv(const DecodeArgs& a, uint32_t dm0, uint32_t dm1, const uint16_t* z, int64_t batch,
                   const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias, uint16_t* y, int64_t n,
                   hipStream_t s) {
-  for (int64_t b0 = 0; b0 < batch; b0 += 8) {
-    const int nb = (int)(batch - b0 < 8 ? batch - b0 : 8);
-    const uint16_t* zb = z + b0 * a.d;
-    uint16_t* yb = y + b0 * n;
-    if (nb == 1) launch_generic_gemv<BITS, 1>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
-    else if (nb <= 4) launch_generic_gemv<BITS, 4>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
-    else launch_generic_gemv<BITS, 8>(a, dm0, dm1, zb, nb, scales, codebook, bias, yb, n, s);
-  }
+  if (batch == 1) launch_generic_gemv<BITS, 1>(a, dm0, dm1, z, batch, scales, codebook, bias, y, n, s);
+  else if (batch <= 4) launch_generic_gemv<BITS, 4>(a, dm0, dm1, z, batch, scales, codebook, bias, y, n, s);
+  else launch_generic_gemv<BITS, 8>(a, dm0, dm1, z, batch, scales, codebook, bias, y, n, s);
 }
 
 inline int make_decode_args(const uint8_t* path, int64_t path_stride, const uint8_t* member,
