@@ -195,9 +195,10 @@ def test_fused_forward_matches_oracle(cuda, n, d, bits, batch):
 # Prompt GEMM: one row tile and one column tile short of every tile the
 # planner takes (128 / 256 / 384 rows x 64 / 128 / 256 batch rows), one K part
 # and several (parts that start inside a row's path stream), a single segment
-# of K, rows of no multiple of 8 or 4, Hadamard blocks 2..8192.
+# of K, rows of no multiple of 8 or 4, Hadamard blocks 2..16384.
 PREFILL_CASES = [  # n, d, bits, S, batch
     (33, 64, 3, 64, 33), (17, 576, 2, 16, 40), (129, 320, 4, 4, 65), (1000, 1030, 3, 8, 67), (64, 8192, 3, 64, 40),
+    (40, 16384, 2, 64, 35), (24, 24576, 4, 16, 70),
     (306, 1280, 2, 64, 115), (1001, 2560, 3, 64, 130), (1536, 9728, 4, 64, 96), (2863, 5120, 3, 64, 193),
     (3000, 1024, 3, 16, 1100), (4097, 768, 2, 4, 1000), (7000, 512, 4, 64, 1537), (9001, 64, 3, 64, 1500),
 ]
@@ -245,7 +246,7 @@ def test_prompt_forward_in_pieces(cuda, monkeypatch):
 
 
 @pytest.mark.parametrize("n,d,bits,batch", [(512, 1024, 2, 17), (511, 1024, 2, 17), (600, 4096, 3, 31), (1000, 2560, 4, 32),
-                                            (513, 1030, 3, 24), (3449, 9728, 3, 17), (3450, 9728, 2, 32)])
+                                            (513, 1030, 3, 24), (512, 8192, 3, 18), (3449, 9728, 3, 17), (3450, 9728, 2, 32)])
 def test_forward_of_17_to_32_rows(cuda, n, d, bits, batch):
     """17..32 rows on both sides of the sizes that take the prompt GEMM."""
     from turbopress_amd.runtime import PackedTCQLinear
