@@ -58,6 +58,15 @@ inline int trellis_taps(int n_states, TrellisTaps* t) {
   return TP_OK;
 }
 
+// Between LDS writes by some lanes of a wave and reads, or writes again, of the
+// same words by others: the compiler keeps them in order (a lane by itself
+// never touches the other lanes' words, so without it they may be swapped).
+// No instruction: one wave's LDS operations execute in order.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ float h2f(uint16_t h) {
   return __half2float(__ushort_as_half(h));
 }

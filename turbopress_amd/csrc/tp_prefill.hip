@@ -128,6 +128,7 @@ __device__ __forceinline__ void pre_write(const PrefillArgs& a, const float16_t 
                     pack_h2(acc[g][c][4 * k + 2] * s2, acc[g][c][4 * k + 3] * s3)};
     }
   }
+  wave_lds_fence();
   const int nb = min(32 * NG, a.batch - b0), nr = min(32 * MG, a.n - row0);
   uint16_t* y0 = a.y + (size_t)b0 * a.ldy + row0;
   // the biases of a lane's 8 rows (its rows repeat: 64 is a multiple of the
@@ -415,6 +416,7 @@ __global__ void __launch_bounds__(256) prefill_reduce_kernel(const PrefillArgs a
   const int row = row0 + (lane & 31);
   const uint16_t* src = lane < 32 ? a.scales : a.bias;
   rows[lane] = src && row < a.n ? gld(src + row) : (uint16_t)0;
+  wave_lds_fence();
   pre_write<1, 1>(a, v, red_out[threadIdx.x >> 6], rows, a.bias ? rows + 32 : nullptr, row0, b0, lane);
 }
 

@@ -214,6 +214,7 @@ viterbi_kernel(const float* __restrict__ z, int64_t ldz, int64_t n, int d, const
           float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, c), K == 2 ? 0x4E : 0x1B, 0xF, 0xF, true));
       cost[64 * q + lane] = f2_t{c, o};
     }
+    wave_lds_fence();
     f2_t next[m];
 #pragma unroll
     for (int ph = 0; ph < m; ++ph) next[ph] = rd[ph][4 * ph];
@@ -249,6 +250,7 @@ viterbi_kernel(const float* __restrict__ z, int64_t ldz, int64_t n, int d, const
       if constexpr (m > 5) column(std::integral_constant<int, 5 % m>{});
       __builtin_amdgcn_sched_barrier(0);
     }
+    wave_lds_fence();  // (before the next block's costs)
   };
   int tb = 0;
   for (; tb + kVitBlock <= d; tb += kVitBlock) block(tb, std::false_type{});
