@@ -99,6 +99,16 @@ def test_tiled_mode_matches_oracle(cuda, bits, n, d, batch):
     assert np.all(np.abs(y - ref) <= bound)
 
 
+@pytest.mark.parametrize("batch", [1, 16, 17])
+def test_tiled_mode_refuses_row_tiles_of_zero_rows(cuda, batch):
+    """tile_rows=0 raises on every forward, as the tile loop of
+    runtime.py:326-331 does, whether or not the rows run through it."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    lin = PackedTCQLinear(make_payload(48, 64, 3, 64, seed=1), mode="tiled", tile_rows=0)
+    with pytest.raises(ValueError):
+        lin(make_activation(batch, 64, seed=1).to(cuda))
+
+
 def test_fwht_scale_rejects_bad_block(cuda):
     from turbopress_amd.hip_kernel import fwht_scale
     x = torch.zeros(1, 96, dtype=torch.float16, device=cuda)

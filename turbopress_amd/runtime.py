@@ -13,8 +13,11 @@ Modes (runtime.py:67):
                     the reference keep working; no Triton code exists here.
   * ``"cached"`` -- load-time decompression: decode + fold the rotation back
                     into fp16 weights with HIP kernels, then a library GEMM.
-  * ``"tiled"``  -- packed streams resident; each forward decodes 1024-row
-                    tiles with the HIP decode kernel and multiplies them.
+  * ``"tiled"``  -- packed streams resident; a forward of more than 16 rows
+                    decodes tiles of ``tile_rows`` weight rows with the HIP
+                    decode kernel and multiplies them, fewer rows multiply
+                    straight from the streams (``tile_rows`` bounds nothing
+                    there: no decoded weights are held).
 
 Every mode computes on the GPU.  A payload on the CPU is moved to the current
 ROCm device at construction; a CPU activation raises RuntimeError -- there is
@@ -216,13 +219,15 @@ class PackedTCQLinear(nn.Module):
             return y.to(x.dtype)
         if self.tiled_packed is not None:
             return hk.forward_tiled(self, x).to(x.dtype)
+        # (a tile_rows of 0 raises here, also where no row tiles are decoded)
+        tiles = None if self._packed_path else range(0, self.out_features, self.tile_rows)
         z = hk.fwht_scale(x, self.rot_scale, self.block)
-        if self._packed_path or z.numel() <= _TILED_GEMV_ROWS * self.in_features:
+        if tiles is None or z.numel() <= _TILED_GEMV_ROWS * self.in_features:
             y = hk.packed_gemv(z, self, bias=self.bias)
-        else:  # tiled
+        else:
             flat = z.reshape(-1, self.in_features)
             y = torch.empty(flat.shape[0], self.out_features, dtype=torch.float16, device=z.device)
-            for r0 in range(0, self.out_features, self.tile_rows):
+            for r0 in tiles:
                 r1 = min(r0 + self.tile_rows, self.out_features)
                 y[:, r0:r1] = flat @ self.decode_rows(r0, r1).T
             y = y.reshape(*z.shape[:-1], self.out_features)
