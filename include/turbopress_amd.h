@@ -218,6 +218,12 @@ int tp_packed_linear_forward_noalloc(const uint16_t* x, int64_t ldx, int64_t bat
  * take: batch outside [1, 65535], d above 2^20, n above 2^24).  Host only. */
 int64_t tp_prefill_workspace_bytes(int64_t n, int64_t d, int64_t batch, int bits);
 
+/* Host only: the tiles tp_packed_linear_prefill takes for a batch on a device
+ * of `cus` compute units: out[0..3] = weight rows and batch rows per tile, K
+ * parts, workgroups.  No reference counterpart: it reports the library's
+ * planning (tests and tuning). */
+int tp_prefill_plan(int64_t n, int64_t d, int64_t batch, int bits, int cus, int64_t* out);
+
 /* tp_packed_linear_forward for a whole prompt (meant for batch > 32): x
  * (contiguous fp16 [batch, d]) is rotated once into the workspace (with
  * rot_scale = NULL and block = 1: x is z already), then a GEMM decodes each

@@ -180,6 +180,14 @@ static void argument_cases() {
   EXPECT(tp_prefill_workspace_bytes(33, INT64_MAX, 33, 3) == 0);
   for (int64_t batch : {33, 199, 2048, 65535})
     for (int64_t n : {33, 2560, 9728}) EXPECT(tp_prefill_workspace_bytes(n, 9728, batch, 3) >= batch * 9728 * 2);
+  int64_t plan[4] = {1, 1, 1, 1};
+  EXPECT(tp_prefill_plan(9728, 2560, 2048, 3, 256, nullptr) == TP_ERR_NULL_POINTER);
+  EXPECT(tp_prefill_plan(33, INT64_MAX, 33, 3, 256, plan) == TP_ERR_BAD_DIMS && plan[0] == 0);
+  EXPECT(tp_prefill_plan(9728, 2560, 2048, 3, 0, plan) == TP_ERR_BAD_DIMS);
+  EXPECT(tp_prefill_plan(9728, 2560, 65536, 3, 256, plan) == TP_ERR_BAD_DIMS);
+  for (int64_t n : {int64_t(1), int64_t(9728), int64_t(1) << 24})
+    for (int64_t d : {int64_t(1), int64_t(9728), int64_t(1) << 20})
+      EXPECT(tp_prefill_plan(n, d, 65535, 4, 256, plan) == TP_OK && plan[2] >= 1 && plan[3] >= plan[2]);
   EXPECT(tp_packed_linear_prefill(nullptr, 64, h, 256, b, b, h, h, nullptr, 16, 256, 3, 64, o, 16, o, 1 << 20,
                                   nullptr) == TP_ERR_NULL_POINTER);
   EXPECT(tp_packed_linear_prefill(h, 64, h, 256, b, b, h, h, nullptr, 16, 256, 9, 64, o, 16, o, 1 << 20, nullptr) ==

@@ -209,3 +209,25 @@ def test_linear_planner_cuts_at_the_qwen3_4b_shapes(built_lib):
     assert o["kparts"] == 1 and o["workgroups"] == 160
     assert _plan(lib, [2560], 9728, 512, 4, ws=0)["kparts"] == 0  # no workspace: the split-K kernel
     assert _plan(lib, [2560], 9728, 512, 9)["kparts"] == 0
+
+
+def test_prefill_planner_tiles(built_lib):
+    """The prompt GEMM's plan on a 256-CU device (host only): long prompts take
+    large tiles in one K part, launches whose tiles leave CUs idle cut K (fewer
+    parts on a smaller device), sizes outside the kernel's range are refused."""
+    from turbopress_amd import _lib
+    out = (ctypes.c_int64 * 4)()
+
+    def plan(n, d, batch, bits=3, cus=256):
+        assert built_lib.tp_prefill_plan(n, d, batch, bits, cus, out) == 0
+        return tuple(out)
+
+    assert plan(9728, 2560, 2048) == (128, 256, 1, 608)
+    assert plan(9728, 2560, 1024) == (384, 128, 1, 208)
+    assert plan(2560, 4096, 199) == (128, 64, 3, 240)
+    assert plan(2560, 9728, 2048)[:3] == (128, 256, 1)
+    assert plan(2560, 4096, 199, cus=64)[2] <= 3
+    for n, d, batch, bits in ((0, 64, 33, 3), (64, 0, 33, 3), (64, 64, 0, 3), (64, 64, 65536, 3), (64, 64, 33, 5),
+                              ((1 << 24) + 1, 64, 33, 3), (64, (1 << 20) + 1, 33, 3)):
+        assert built_lib.tp_prefill_plan(n, d, batch, bits, 256, out) != 0 and list(out) == [0, 0, 0, 0]
+    assert built_lib.tp_prefill_plan(64, 64, 33, 3, 256, None) == _lib.TP_ERR_NULL_POINTER

@@ -192,10 +192,9 @@ def test_fused_forward_matches_oracle(cuda, n, d, bits, batch):
     assert O.max_rel(y, O.tiled_forward(payload_numpy(p), x.numpy())) <= GEMV_TOL
 
 
-# Prompt GEMM: one row tile and one column tile short of every tile the
-# planner takes (128 / 256 / 384 rows x 64 / 128 / 256 batch rows), one K part
-# and several (parts that start inside a row's path stream), a single segment
-# of K, rows of no multiple of 8 or 4, Hadamard blocks 2..16384.
+# Prompt GEMM through its whole range of sizes: a single segment of K and
+# long rows, ragged last tiles, rows of no multiple of 8 or 4, Hadamard blocks
+# 2..16384, every trellis (each tile and K cut: PREFILL_PLANS below).
 PREFILL_CASES = [  # n, d, bits, S, batch
     (33, 64, 3, 64, 33), (17, 576, 2, 16, 40), (129, 320, 4, 4, 65), (1000, 1030, 3, 8, 67), (64, 8192, 3, 64, 40),
     (40, 16384, 2, 64, 35), (24, 24576, 4, 16, 70),
@@ -229,6 +228,80 @@ def test_prompt_forward_matches_oracle_deterministically(cuda, n, d, bits, n_sta
     out = guard[:batch * n].view(batch, n)
     assert hk.forward_prefill(lin, xd, out, lin.bias)
     assert torch.equal(out, y) and bool((guard[batch * n:] == 7.0).all())
+
+
+# Each tile of the prompt GEMM (weight rows x batch rows), with one K part and
+# with several where the planner cuts K, as it takes them on 256 CUs: (n, d,
+# batch) -> (weight rows, batch rows, K parts).  Ragged in all three, at least
+# four half steps per K part, so that each of the three z buffers is refilled.
+# Every rate: the waits between weight and z loads depend on (rate, tile).
+PREFILL_PLANS = [
+    ((181, 516, 41), (128, 64, 1)), ((45, 2308, 34), (128, 64, 10)),
+    ((1046, 516, 1810), (128, 128, 1)), ((1046, 5116, 589), (128, 128, 5)),
+    ((3594, 516, 1033), (128, 256, 1)), ((1410, 6148, 1366), (128, 256, 3)),
+    ((7325, 516, 1551), (256, 256, 1)), ((10965, 516, 515), (384, 128, 1)), ((3594, 9732, 515), (384, 128, 5)),
+]
+
+
+def _prefill_plan(n, d, batch, bits=3, cus=256):
+    import ctypes
+    from turbopress_amd import _lib
+    out = (ctypes.c_int64 * 4)()
+    _lib.check(_lib.lib().tp_prefill_plan(n, d, batch, bits, cus, out), "prefill_plan")
+    return tuple(out)
+
+
+@pytest.mark.parametrize("bits,n_states", [(2, 16), (3, 64), (4, 64), (2, 64), (3, 8), (4, 4)])
+@pytest.mark.parametrize("size,tile", PREFILL_PLANS)
+def test_every_prompt_tile(cuda, size, tile, bits, n_states):
+    """Every (tile, K cut, rate) against the fp64 product of the weights that
+    the natural-stream kernel decodes and the row-major rotation (both
+    bit-exact with the oracle in their own tests), each output row and column
+    relative to its own largest values: the sum and the sum with the bias are
+    each rounded to fp16, 2^-11 of either; the fp32 sums' own rounding is far
+    below the 5 % of that allowed for it."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    (n, d, batch), cus = size, torch.cuda.get_device_properties(cuda).multi_processor_count
+    if cus == 256:
+        assert _prefill_plan(n, d, batch, bits)[:3] == tile
+    p = make_payload(n, d, bits, n_states, seed=n + bits, bias=True)
+    lin = PackedTCQLinear(p, mode="hip")
+    x = make_activation(batch, d, seed=batch).to(cuda)
+    y = lin(x).double()
+    levels = hk.window_decode_levels(p["path_packed"].to(cuda), p["member_packed"].to(cuda), d, bits, n_states)
+    w = lin.codebook.double()[levels.long()] * lin.scales.double()[:, None]
+    sums = hk.fwht_scale(x, lin.rot_scale, lin.block).double() @ w.T
+    ref = sums + lin.bias.double()
+    err = (y - ref).abs()
+    for axis in (0, 1):
+        bound = 2.0 ** -11 * 1.05 * (sums.abs().amax(axis) + ref.abs().amax(axis))
+        assert bool((err.amax(axis) <= bound).all()), axis
+
+
+@pytest.mark.parametrize("n,d,batch", [(600, 4096, 199), (1046, 516, 70), (512, 1024, 20)])
+def test_prompt_forward_replays_from_a_graph(cuda, n, d, batch):
+    """A captured prompt (K parts, one part, and 17..32 rows), its workspace
+    from the graph's pool: every replay, with other work and new inputs in
+    between, equals the eager call."""
+    from turbopress_amd.runtime import PackedTCQLinear
+    lin = PackedTCQLinear(make_payload(n, d, 3, 64, seed=n, bias=True), mode="hip")
+    x = make_activation(batch, d, seed=1).to(cuda)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        lin(x)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        y = lin(x)
+    for seed in (1, 2, 3):
+        x.copy_(make_activation(batch, d, seed=seed))
+        want = lin(x)
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want), seed
 
 
 def test_prompt_forward_in_pieces(cuda, monkeypatch):

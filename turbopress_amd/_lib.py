@@ -55,6 +55,7 @@ SIGNATURES: dict[str, tuple] = {
     "tp_packed_linear_forward_noalloc": (c_int, [_P, _I64, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64,
                                                  c_int, c_int, _P, _I64, _P]),
     "tp_prefill_workspace_bytes": (c_int64, [_I64, _I64, _I64, c_int]),
+    "tp_prefill_plan": (c_int, [_I64, _I64, _I64, c_int, c_int, POINTER(c_int64)]),
     "tp_packed_linear_prefill": (c_int, [_P, _I64, _P, _I64, _P, _P, _P, _P, _P, _I64, _I64, c_int, c_int,
                                          _P, _I64, _P, _I64, _P]),
     "tp_packed_linear_forward_group": (c_int, [c_int, _P, _I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P,

@@ -519,6 +519,21 @@ extern "C" int64_t tp_prefill_workspace_bytes(int64_t n, int64_t d, int64_t batc
   return pre_workspace(plan_prefill(n, 2 * g.G4, batch, device_cu_count()), 2 * g.G4);
 }
 
+extern "C" int tp_prefill_plan(int64_t n, int64_t d, int64_t batch, int bits, int cus, int64_t* out) {
+  if (!out) return TP_ERR_NULL_POINTER;
+  for (int i = 0; i < 4; ++i) out[i] = 0;
+  if (cus < 1) return TP_ERR_BAD_DIMS;
+  Geom g;
+  const int st = pre_geom(n, d, batch, bits, &g);
+  if (st) return st;
+  const PrePlan p = plan_prefill(n, 2 * g.G4, batch, cus);
+  out[0] = 32 * kPreWM * p.mg;
+  out[1] = 64 * p.ng;
+  out[2] = p.kparts;
+  out[3] = p.rb * p.cb * p.kparts;
+  return TP_OK;
+}
+
 extern "C" int tp_packed_linear_prefill(const uint16_t* x, int64_t batch, const uint16_t* rot_scale, int64_t block,
                                         const uint8_t* path_tiled, const uint8_t* member_tiled,
                                         const uint16_t* scales, const uint16_t* codebook, const uint16_t* bias,
