@@ -18,7 +18,7 @@
 //
 // Calling the 32-row kernels once per 32 rows decodes every weight again for
 // each of them: 1316 us for 2048 rows of a 9728 x 2560 linear (k=3) and 122 us
-// for 199 rows of 2560 x 4096, against 128 and 25 us here.
+// for 199 rows of 2560 x 4096, against 125-132 and 23-25 us here.
 //
 // What bounds the GEMM: at 2048 x 2560 x 9728 the launch takes 112-130 us
 // (0.79-0.91 PFLOP/s; a dense fp16 library product of that shape 103-117 us on
@@ -131,8 +131,7 @@ __device__ __forceinline__ void pre_write(const PrefillArgs& a, const float16_t 
   wave_lds_fence();
   const int nb = min(32 * NG, a.batch - b0), nr = min(32 * MG, a.n - row0);
   uint16_t* y0 = a.y + (size_t)b0 * a.ldy + row0;
-  // the biases of a lane's 8 rows (its rows repeat: 64 is a multiple of the
-  // chunks of a batch row, except for MG = 3)
+  // 8 rows' sums, rounded, plus their biases
   auto add_bias = [&](u32x4_t w, int r) __attribute__((always_inline)) {
     const u32x4_t bw = *reinterpret_cast<const u32x4_t*>(br + r);
 #pragma unroll
@@ -433,14 +432,19 @@ constexpr int kPreMaxParts = 16;
 // The cheapest of five tiles and 1..16 K parts in a model of the launch: per
 // round of one workgroup per CU 7 us (table, first loads, output) plus the
 // half steps of a part, and for several parts the second launch, 4 us plus
-// its traffic at 4 TB/s.  us per half step by tile, from launches that fill
-// the chip: 256 x 256 1.70, 384 x 128 1.25, 128 x 256 0.76, 128 x 128 0.46,
-// 128 x 64 0.30.  Against forced plans (k=3, total with the rotation):
-// 9728 x 2560 at 2048 rows 128 x 256 140 us (256 x 256 168, 384 x 128 142,
-// 128 x 128 162), at 1024 rows 384 x 128 78 us (128 x 256 92); 2560 x 9728 at
-// 2048 rows 128 x 256 180 us (256 x 256 in 3 parts 181, in one part 259);
-// 2560 x 4096 at 199 rows 128 x 64 in 3 parts 37 us (128 x 128 in 4 parts 38,
-// 128 x 64 in one part 45).
+// its traffic at 4 TB/s.  What decides is the tiles' ratio, not the scale: the
+// model's us per half step are 256 x 256 1.70, 384 x 128 1.25, 128 x 256 0.76,
+// 128 x 128 0.46, 128 x 64 0.30; the launches alone, 16 x 16 tiles of each, a
+// dozen in a row, k=3, take 2.00 / 1.57 / 1.03 / 0.59 / 0.43 and 1-7 us
+// besides.  The pick against the fastest of all forced plans (k=3, with the
+// rotation): 9728 x 2560 at 2048 rows 128 x 256 125 us (fastest; 384 x 128 133,
+// 256 x 256 139, 128 x 128 141), at 1024 rows 384 x 128 67.4 (256 x 256 67.2,
+// 128 x 256 79.6); 4096 x 2560 at 2048 rows 128 x 256 55.7 (fastest); 2560 x
+// 9728 at 2048 rows 128 x 256 in one part 151 (256 x 256 in 3 parts 145: 160
+// workgroups leave 96 CUs idle, and the model takes K parts to cost more than
+// they do), at 512 rows 128 x 128 in 3 parts 48.4 (128 x 256 in 6 parts 47.1);
+// 2560 x 4096 at 199 rows 128 x 64 in 3 parts 24.4 (fastest; 128 x 128 in 4
+// parts 24.9, 128 x 64 in one part 32.5).
 PrePlan plan_prefill(int64_t n, int64_t U, int64_t batch, int cus) {
   static constexpr struct {
     int mg, ng;

@@ -44,9 +44,12 @@ struct RotRows {
 // 4096 take the four waves of a workgroup, 4096 columns, together.  The
 // scales of its columns stay in registers and the next row loads while this
 // one is transformed.  Columns past d load as zeros, are whole blocks, and
-// come out as the zeros that pad a row to `ld`.  Bound by memory traffic
-// (x in, z out): 2048 x 9728 (block 512) 21.5 us = 3.7 TB/s, 8192 x 4096
-// (block 4096) 33.7 us = 4.0 TB/s.  The general kernel (one workgroup per
+// come out as the zeros that pad a row to `ld`.  Row-major it is bound by VALU
+// issue (products, butterflies, lane moves): 77 / 83 / 68 % of the SIMD cycles
+// of resident workgroups at 2048 x 2560 and 2048 x 9728 (block 512) and 8192 x
+// 4096 (block 4096), 8.2 / 21.8 / 37.5 us where a copy takes 3.9 / 12.3 / 19.6.
+// In operand order the stores of a wave are 16-byte pieces of 32 cache lines
+// and weigh more the larger z is: 12.9 / 39.8 / 66.5 us.  The general kernel (one workgroup per
 // block and row, every stage above 8 columns through LDS) took 24.7 us for
 // 2048 x 2560 (block 512; here 9.0) and 16.4 us for 199 x 4096 (block 4096;
 // here 4.5), and 68.6 us for the load-time fold of a 2560 x 9728 weight

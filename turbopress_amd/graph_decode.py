@@ -9,13 +9,14 @@ cache the two produce the same greedy tokens.  Every PackedTCQLinear forward
 is capture-safe (no host synchronisation, no allocation outside torch's
 graph pool).
 
-The prefill runs the prompt as one batch.  Above 8 rows the batched
-decode-GEMV splits K over workgroups and adds their fp32 partial sums with
-atomics in arrival order (as the reference's split-D configurations do,
-``turbopress/triton_kernel.py:126-129``), so two prefills of one prompt can
-differ in the last bits of the cache -- enough to flip a greedy token where
-the top two logits nearly tie.  ``prefill`` therefore runs once and both
-loops start from copies of its cache.  The batch-1 decode steps add in a
+The prefill runs the prompt as one batch.  Prompts of 9..32 tokens mostly run
+the batched decode-GEMV, which splits K over workgroups and adds their fp32
+partial sums with atomics in arrival order (as the reference's split-D
+configurations do, ``turbopress/triton_kernel.py:126-129``), so two prefills of
+such a prompt can differ in the last bits of the cache -- enough to flip a
+greedy token where the top two logits nearly tie.  (Longer prompts run the
+prompt GEMM, which adds in a fixed order.)  ``prefill`` therefore runs once and
+both loops start from copies of its cache.  The batch-1 decode steps add in a
 fixed order: their tokens are reproducible.
 """
 

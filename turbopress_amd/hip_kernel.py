@@ -120,7 +120,10 @@ def packed_gemv(z: Tensor, layer, bias: Tensor | None = None) -> Tensor:
     flat = z.reshape(-1, d).to(torch.float16).contiguous()
     out = torch.empty(flat.shape[0], n, dtype=torch.float16, device=z.device)
     if getattr(layer, "tiled_packed", None) is not None:
-        # (rows of no multiple of 4 columns would be laid out column by column)
+        # (rows of no multiple of 4 columns would be laid out column by column: at
+        # 2048 rows of 700 x 9727 that and the GEMM take 4230 us, this 984; forward
+        # rotates such rows column by column either way and takes the GEMM: 4230
+        # against 5149)
         if flat.shape[0] > 32 and d % 4 == 0 and forward_prefill(layer, flat, out, bias, rotated=True):
             return out.reshape(*z.shape[:-1], n)
         ldz = layer._tiled_geo["z_cols"]
@@ -259,7 +262,9 @@ def rotate_padded(x: Tensor, rot_scale: Tensor, block: int, ldz: int) -> Tensor:
 
 
 def gemv_tiled(zpad: Tensor, layer, bias: Tensor | None, out: Tensor) -> Tensor:
-    """out[B, n] = packed GEMV over the device layout; zpad fp16 [B, ldz]."""
+    """out[B, n] = packed GEMV over the device layout; zpad fp16 [B, ldz].
+    (More than 32 rows come here only from packed_gemv with d % 4, or for
+    sizes the prompt GEMM does not take.)"""
     n, d = layer.out_features, layer.in_features
     buf = layer.tiled_packed
     pb = layer._tiled_geo["path_bytes"]
@@ -314,24 +319,32 @@ def forward_prefill(layer, flat: Tensor, y: Tensor, bias: Tensor | None, rotated
 
 
 def forward_tiled(layer, x: Tensor) -> Tensor:
-    """Rotation + decode-GEMV + bias: more than 16 rows run the prompt GEMM
-    (forward_prefill); fewer one fused launch (tp_packed_linear_forward)
-    when the rotation fits the launch (up to 8 rows, or Hadamard blocks <=
-    512), otherwise the rows rotate once into the padded layout and run the
-    batched decode-GEMV (tp_tcq_gemv_tiled).  fp16 [..., n]."""
+    """Rotation + decode-GEMV + bias: more than 32 rows run the prompt GEMM
+    (forward_prefill), 17..32 rows where the rule below says so; fewer one
+    fused launch (tp_packed_linear_forward) when the rotation fits the launch
+    (up to 8 rows, or Hadamard blocks <= 512), otherwise the rows rotate once
+    into the padded layout and run the batched decode-GEMV
+    (tp_tcq_gemv_tiled).  fp16 [..., n]."""
     _require_cuda(x, "x")
     n, d = layer.out_features, layer.in_features
     flat = x.reshape(-1, d).to(torch.float16).contiguous()
     rows = flat.shape[0]
     y = torch.empty(rows, n, dtype=torch.float16, device=x.device)
     # 17..32 rows too where the fused launch does not rotate (Hadamard blocks
-    # above 512) or decodes 2^25 weights or more: 32 rows of 2560 x 4096 (block
-    # 4096) 19.5 -> 15.9 us of GPU time and 32.2 -> 23.5 us per eager call, 4096
-    # x 9728 27.5 -> 23.0 per call.  Below that the one launch is cheaper to call
-    # (9728 x 2560 20.6 against 23.5 us, though 20.6 against 16.6 of GPU time),
-    # with few rows of weights K parts leave the GEMM short of workgroups (300 x
-    # 9216: 15.4 against 17.7), and 9..16 rows fill half of its columns (16 rows
-    # of 2560 x 4096: 15.1 against 15.7).
+    # above 512) or decodes 2^25 weights or more.  The lines lie where a call
+    # costs the same from Python, not the GPU.  us of GPU time at 17 / 24 / 32
+    # rows, and per eager call at 32, GEMM against the other path:
+    #   512 x 1024   12.6 / 12.7 / 12.7 against 13.9 / 14.5 / 15.2, 17.6 against 26.3
+    #   512 x 9216   17.1 / 17.0 / 17.1 against 15.9 / 16.2 / 17.1, 20.6 against 26.5
+    #   448 x 4096   15.7 / 15.7 / 15.8 against 14.4 / 14.7 / 15.6, 20.4 against 25.7
+    #   2560 x 4096  15.7 / 15.8 / 15.8 (with the row-by-row rotation 27.7 / 28.4 / 29.6)
+    #   9728 x 2560  16.8 / 16.8 / 16.8 against 18.3 / 19.2 / 20.4, 20.0 against 20.6
+    #   13056 x 2560 21.5 / 21.4 / 21.4 against 20.4 / 21.3 / 22.6, 21.8 against 22.8
+    #   13120 x 2560 21.5 / 21.4 / 21.4 against 28.4 / 29.1 / 30.6 (2^25 weights)
+    #   3440 x 9728  20.5 / 20.5 / 20.5 against 31.0 / 32.3 / 33.6: below 2^25,
+    # so long rows just under the line, and captured calls, pay for the rule.
+    # 9..16 rows fill half of the GEMM's columns (512 x 4096, 16 rows: 15.6
+    # against 13.0).
     if rows > 16 and (rows > 32 or n >= 512 and (layer.block > 512 or n * d >= 1 << 25)) \
             and forward_prefill(layer, flat, y, layer.bias):
         return y.reshape(*x.shape[:-1], n)
@@ -346,6 +359,7 @@ def forward_tiled(layer, x: Tensor) -> Tensor:
     bias = layer.bias
     stream = current_stream_ptr(x.device)
     lib = _lib.lib()
+    # (more than one piece only for sizes the GEMM does not take: d > 2^20, n > 2^24)
     for b0 in range(0, rows, 32):
         nb = min(32, rows - b0)
         ws, ws_bytes = layer_workspace(layer, nb)

@@ -39,10 +39,12 @@ __all__ = ["PackedTCQLinear", "MODES", "Trellis", "trellis_generators", "pack_li
 MODES = ("hip", "triton", "cached", "tiled")
 
 # Rows up to which mode "tiled" multiplies straight from the packed streams
-# (one launch, weights unrounded) instead of decoding row tiles: one pass of
-# the natural-stream GEMV per 8 rows.  16 rows: 9728 x 2560 48 us (row tiles
-# 396), 4096 x 9728, k=4, 71 us (168); at 32 rows of the latter 136 us, which a
-# larger tile_rows than the default 1024 can beat.
+# (one launch, weights unrounded) instead of decoding row tiles into fp16
+# weights for a library product.  us per eager call at 16 / 32 rows, streams
+# against row tiles of 1024 and against one tile of all rows: 3072 x 1024 28 /
+# 27 against 133 and 57; 9728 x 2560 37 / 66 against 396 and 56; 4096 x 9728,
+# k=4, 62 / 105 against 172 and 57.  Above 16 rows a tile_rows larger than the
+# default wins on large linears.
 _TILED_GEMV_ROWS = 16
 
 _GENERATORS = {4: (0o5, 0o7), 8: (0o15, 0o17), 16: (0o23, 0o35), 64: (0o133, 0o171)}
