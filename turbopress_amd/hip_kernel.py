@@ -331,20 +331,24 @@ def forward_tiled(layer, x: Tensor) -> Tensor:
     rows = flat.shape[0]
     y = torch.empty(rows, n, dtype=torch.float16, device=x.device)
     # 17..32 rows too where the fused launch does not rotate (Hadamard blocks
-    # above 512) or decodes 2^25 weights or more.  The lines lie where a call
-    # costs the same from Python, not the GPU.  us of GPU time at 17 / 24 / 32
+    # above 512) or decodes 2^25 weights or more.  us of GPU time at 17 / 24 / 32
     # rows, and per eager call at 32, GEMM against the other path:
-    #   512 x 1024   12.6 / 12.7 / 12.7 against 13.9 / 14.5 / 15.2, 17.6 against 26.3
-    #   512 x 9216   17.1 / 17.0 / 17.1 against 15.9 / 16.2 / 17.1, 20.6 against 26.5
-    #   448 x 4096   15.7 / 15.7 / 15.8 against 14.4 / 14.7 / 15.6, 20.4 against 25.7
-    #   2560 x 4096  15.7 / 15.8 / 15.8 (with the row-by-row rotation 27.7 / 28.4 / 29.6)
-    #   9728 x 2560  16.8 / 16.8 / 16.8 against 18.3 / 19.2 / 20.4, 20.0 against 20.6
-    #   13056 x 2560 21.5 / 21.4 / 21.4 against 20.4 / 21.3 / 22.6, 21.8 against 22.8
-    #   13120 x 2560 21.5 / 21.4 / 21.4 against 28.4 / 29.1 / 30.6 (2^25 weights)
-    #   3440 x 9728  20.5 / 20.5 / 20.5 against 31.0 / 32.3 / 33.6: below 2^25,
-    # so long rows just under the line, and captured calls, pay for the rule.
-    # 9..16 rows fill half of the GEMM's columns (512 x 4096, 16 rows: 15.6
-    # against 13.0).
+    #   block > 512, two launches, so the GEMM is the cheaper eager call throughout:
+    #     300 x 9216   17.3 / 17.4 / 17.6 against 15.2 / 15.4 / 15.7, 20.3 against 26.1
+    #     512 x 4096   15.8 / 15.8 / 15.8 against 14.6 / 15.0 / 15.7, 20.4 against 26.4
+    #     512 x 1024   12.6 / 12.7 / 12.7 against 13.9 / 14.5 / 15.2, 17.6 against 26.3
+    #     1024 x 4096  15.3 / 15.5 / 15.4 against 15.9 / 16.0 / 17.2, 20.6 against 26.2
+    #     2560 x 4096  15.8 / 15.9 / 16.0 against 17.4 / 18.3 / 19.6, 20.2 against 25.8
+    #   block <= 512, one fused launch:
+    #     1536 x 576   11.0 / 11.1 / 11.1 against 12.2 / 13.0 / 14.4, 17.4 against 15.8
+    #     9728 x 2560  16.8 / 16.8 / 16.8 against 18.3 / 19.2 / 20.4, 20.0 against 20.6
+    #     13056 x 2560 21.5 / 21.4 / 21.4 against 20.4 / 21.3 / 22.6, 21.8 against 22.8
+    #     13120 x 2560 21.5 / 21.4 / 21.4 against 28.4 / 29.1 / 30.6 (2^25 weights)
+    #     3440 x 9728  20.5 / 20.5 / 20.5 against 31.0 / 32.3 / 33.6 (below 2^25)
+    # n = 512 is where the GPU times of the first kind meet.  2^25 is where most
+    # eager calls of the second kind do; captured ones, and long rows below it,
+    # pay for that line.  9..16 rows fill half of the GEMM's columns (512 x
+    # 4096, 16 rows: 15.6 against 13.0).
     if rows > 16 and (rows > 32 or n >= 512 and (layer.block > 512 or n * d >= 1 << 25)) \
             and forward_prefill(layer, flat, y, layer.bias):
         return y.reshape(*x.shape[:-1], n)
